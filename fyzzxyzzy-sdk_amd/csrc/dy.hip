@@ -55,20 +55,20 @@ constexpr int kPgsBlocks = 256;       // workgroups of the sweep (no grid barrie
 enum : u32 { kFront0 = 0, kFront1, kFront2, kPend, kNParts, kPosIters, kVelIters, kRounds, kContacts, kFrictionRows,
              kNbWord, kCtrWords = 16 };
 
-// one contact row (SolverContactPoint fields the solve reads), 64 B
-struct alignas(16) CRow {
-    float nx, ny, nz, vm;
-    float rax, ray, raz, biased;
-    float rbx, rby, rbz, unbiased;
-    float applied, max_impulse, pad0, pad1;
-};
-// one friction row (SolverContactFriction), 64 B
-struct alignas(16) FRow {
-    float tx, ty, tz, vm;
-    float rax, ray, raz, bias;
-    float rbx, rby, rbz, target;
-    float applied, pad0, pad1, pad2;
-};
+// The solver rows of the manager at a partition-sorted position, laid out
+// for the eight lanes that solve it (4 lanes per body: three components and
+// one for scalars): 4 row pairs (contact rows 0/1, 2/3, the friction rows of
+// anchor 0, of anchor 1) of 8 float4, 512 B. Lane q (side q >> 2, component
+// c = q & 3) of pair p holds
+//   c < 3: (direction_c, lever_c) of the pair's first row, then of its
+//          second (direction: contact normal or tangent; lever: the side's
+//          angular part of the row)
+//   c = 3: the scalars of the first row (side 0) or the second (side 1):
+//          contact (velocity multiplier, biased error, unbiased error,
+//          maximum impulse), friction (velocity multiplier, bias, target, 0)
+// so that a pair is one 128-B request of the eight lanes.
+constexpr u32 kRowLanes = 8;       // float4 per row pair
+constexpr u32 kRowQuads = 4 * kRowLanes;  // float4 per manager
 
 struct Ws {
     // step inputs
@@ -99,9 +99,11 @@ struct Ws {
     u32* pos_of;    // [nm] partition-sorted position of each manager in a partition
     uint4* srank;   // [nm] per position: rank of the manager among body0's / body1's (by partition), their degrees
     u32* erank;     // [2 nm] per incidence entry: rank among the body's managers by partition
-    u64* vst;       // [8 nb] sweep state, a 64-byte line per body: (component bits, updates applied) x 6, pad
-    CRow* crow;
-    FRow* frow;
+    u64* vst;       // [8 nb] sweep state, a 64-byte line per body: 4 chunks of (linear bits, updates applied,
+                    // angular bits, updates applied): x, y, z, then the inverse mass
+    float4* rows;   // [32 nm] solver rows by partition-sorted position (kRowQuads each)
+    float* app;     // [8 nm] applied impulses by position: 4 contact rows, 4 friction rows
+    float4* fric;   // [nm] by position: the patch's static and dynamic friction, its flags
     u32 *part_count, *part_off, *part_fill;
     u32* blocksums;
     u32* ctr;
@@ -374,6 +376,7 @@ __global__ __launch_bounds__(kBlock) void k_part_clear(Ws W) {
         W.max_dyn[i] = 0;
 #pragma unroll
         for (u32 k = 0; k < 8; ++k) W.vst[8 * i + k] = 0ull;  // 0.0f, no updates yet
+        W.vst[8 * i + 6] = __float_as_uint(W.lin[i].w);       // the inverse mass (constant through the sweep)
     }
     if (i < kMaxParts) {
         W.part_count[i] = 0;
@@ -834,6 +837,34 @@ struct Run {
     int next;
 };
 
+// A solver row as prepared, and a pair of them in the sweep's lane layout.
+struct RowOut {
+    V d, ra, rb;
+    float4 s;
+};
+__device__ inline void store_rows(float4* o, const RowOut& x, const RowOut& y) {
+    o[0] = make_float4(x.d.x, x.ra.x, y.d.x, y.ra.x);
+    o[1] = make_float4(x.d.y, x.ra.y, y.d.y, y.ra.y);
+    o[2] = make_float4(x.d.z, x.ra.z, y.d.z, y.ra.z);
+    o[3] = x.s;
+    o[4] = make_float4(x.d.x, x.rb.x, y.d.x, y.rb.x);
+    o[5] = make_float4(x.d.y, x.rb.y, y.d.y, y.rb.y);
+    o[6] = make_float4(x.d.z, x.rb.z, y.d.z, y.rb.z);
+    o[7] = y.s;
+}
+// Row r (0-3 contact, 4-7 friction) of a position, read back by one thread.
+__device__ inline RowOut read_row(const Ws& W, u32 pos, u32 r) {
+    const float4* o = W.rows + static_cast<std::size_t>(kRowQuads) * pos + kRowLanes * (r >> 1);
+    const bool second = r & 1u;
+    RowOut v;
+    const float4 x = o[0], y = o[1], z = o[2], bx = o[4], by = o[5], bz = o[6];
+    v.d = second ? V{x.z, y.z, z.z} : V{x.x, y.x, z.x};
+    v.ra = second ? V{x.w, y.w, z.w} : V{x.y, y.y, z.y};
+    v.rb = second ? V{bx.w, by.w, bz.w} : V{bx.y, by.y, bz.y};
+    v.s = o[second ? 7 : 3];
+    return v;
+}
+
 // One thread per manager: materials, same-normal runs, friction-patch
 // correlation with the previous step, contact rows, anchor growth and
 // friction rows (scene.cpp:7794-8505).
@@ -1029,6 +1060,9 @@ __global__ __launch_bounds__(128) void k_prep(Ws W) {
     }
     // contact rows in the correlation-list order (scene.cpp:8204-8225, 8237-8330)
     bool bad = false;
+    const u32 pos = W.pos_of[m];
+    float4* const out = W.rows + static_cast<std::size_t>(kRowQuads) * pos;
+    RowOut r[2];
     for (u32 q = 0; q < no; ++q) {
         const fyzz_dy_contact& C = M.contacts[(order_bits >> (2 * q)) & 3u];
         const V n = header;
@@ -1051,24 +1085,15 @@ __global__ __launch_bounds__(128) void k_prep(Ws W) {
         const float target = target_velocity - vrel;
         const float pen_scaled = separated ? pen_inv_dt : pen * (inv_dt * rigid_contact_bias);
         const float scaled_bias = bouncing ? 0.0f : vm * smax(max_pen_bias, pen_scaled);
-        CRow r;
-        r.nx = n.x;
-        r.ny = n.y;
-        r.nz = n.z;
-        r.vm = vm;
-        r.rax = ra.x;
-        r.ray = ra.y;
-        r.raz = ra.z;
-        r.biased = target * vm - scaled_bias;
-        r.rbx = rb.x;
-        r.rby = rb.y;
-        r.rbz = rb.z;
-        r.unbiased = target * vm - (bouncing ? 0.0f : smax(scaled_bias, 0.0f));
-        r.applied = 0.0f;
-        r.max_impulse = kFltMax;
-        r.pad0 = r.pad1 = 0.0f;
-        bad |= !isfinite(response) || !isfinite(r.biased) || !isfinite(r.unbiased);
-        W.crow[4 * m + q] = r;
+        RowOut& o = r[q & 1u];
+        const float biased = target * vm - scaled_bias;
+        const float unbiased = target * vm - (bouncing ? 0.0f : smax(scaled_bias, 0.0f));
+        o.d = n;
+        o.ra = ra;
+        o.rb = rb;
+        o.s = make_float4(vm, biased, unbiased, kFltMax);
+        bad |= !isfinite(response) || !isfinite(biased) || !isfinite(unbiased);
+        if ((q & 1u) || q + 1 == no) store_rows(out + kRowLanes * (q >> 1), r[0], (q & 1u) ? r[1] : r[0]);
         if (W.tape) {
             // err = target vm - bias with target = -(1 + e) vrel when bouncing, -vrel otherwise
             W.craw[2 * (4 * m + q)] = make_float4(ra_x_n.x, ra_x_n.y, ra_x_n.z, bouncing ? -(1.0f + restitution) : -1.0f);
@@ -1158,27 +1183,19 @@ __global__ __launch_bounds__(128) void k_prep(Ws W) {
                     const V j0 = transform(a, ax0);
                     const V j1 = transform(b, ax1);
                     const float response = (a.inv_mass + vdot(j0, j0)) + (b.inv_mass + vdot(j1, j1));
-                    FRow fr;
-                    fr.tx = tangent.x;
-                    fr.ty = tangent.y;
-                    fr.tz = tangent.z;
-                    fr.vm = response > 0.0f ? rigid_contact_bias / response : 0.0f;
-                    fr.rax = j0.x;
-                    fr.ray = j0.y;
-                    fr.raz = j0.z;
-                    fr.bias = vdot(tangent, err) * inv_dt;
-                    fr.rbx = j1.x;
-                    fr.rby = j1.y;
-                    fr.rbz = j1.z;
-                    fr.target = -(vdot(tangent, rel) + vdot(ax0, a.w) - vdot(ax1, b.w));
-                    fr.applied = 0.0f;
-                    fr.pad0 = fr.pad1 = fr.pad2 = 0.0f;
-                    W.frow[4 * m + 2 * k + ti] = fr;
+                    RowOut& fr = r[ti];
+                    fr.d = tangent;
+                    fr.ra = j0;
+                    fr.rb = j1;
+                    fr.s = make_float4(response > 0.0f ? rigid_contact_bias / response : 0.0f,
+                                       vdot(tangent, err) * inv_dt,
+                                       -(vdot(tangent, rel) + vdot(ax0, a.w) - vdot(ax1, b.w)), 0.0f);
                     if (W.tape) {
                         W.fraw[2 * (4 * m + 2 * k + ti)] = make_float4(ax0.x, ax0.y, ax0.z, 0.0f);
                         W.fraw[2 * (4 * m + 2 * k + ti) + 1] = make_float4(ax1.x, ax1.y, ax1.z, 0.0f);
                     }
                 }
+                store_rows(out + kRowLanes * (2 + k), r[0], r[1]);
             }
         }
     }
@@ -1199,23 +1216,24 @@ __global__ __launch_bounds__(128) void k_prep(Ws W) {
     W.order[m] = no | ((order_bits & 3u) << 8) | ((no > 1 ? (order_bits >> 2) & 3u : 0u) << 12) |
                  ((no > 2 ? (order_bits >> 4) & 3u : 0u) << 16) | ((no > 3 ? (order_bits >> 6) & 3u : 0u) << 20);
     // the sweep reads the row counts with the position record
-    W.sinfo[W.pos_of[m]].w = static_cast<int>(no | (P.anchors << 8));
+    W.sinfo[pos].w = static_cast<int>(no | (P.anchors << 8));
+    W.fric[pos] = make_float4(o.static_friction, o.dynamic_friction, __uint_as_float(o.flags), 0.f);
+    float4* const ap = reinterpret_cast<float4*>(W.app + 8ull * pos);
+    ap[0] = ap[1] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // ------------------------------------------------------------------ solve
 
 // scene.cpp:8985-9010 (normal rows), 9050-9120 (friction rows)
 // Coherent body state: during the sweep a body's velocity change lives in
-// one 64-byte line of three 16-byte chunks, each chunk two components'
-// bits, each followed by the number of updates applied to the body, moved
+// one 64-byte line of four 16-byte chunks (x, y, z, inverse mass), each
+// value followed by the number of updates applied to the body, moved
 // between workgroups on different XCDs by device-coherent (sc1) 16-byte
-// loads and stores (one request per chunk). A reader takes the state when
-// all six counts carry the count it waits for: a count is written once
-// per body, so matching counts give the values written with it, and a
-// writer needs no wait between its state stores and a separate counter.
-struct BodyState {
-    V v, w;
-};
+// loads and stores. The four lanes of a body's side move the whole line as
+// one request. A reader takes the state when all counts carry the count it
+// waits for: a count is written once per body, so matching counts give the
+// values written with it, and a writer needs no wait between its state
+// stores and a separate counter.
 typedef u32 Chunk __attribute__((ext_vector_type(4)));
 constexpr u32 kStateBytes = 64;
 constexpr int kDeviceCoherent = 16;  // cache policy: sc1 (device scope)
@@ -1226,20 +1244,9 @@ __device__ inline __amdgpu_buffer_rsrc_t state_rsrc(const Ws& W) {
 __device__ inline Chunk load_chunk(__amdgpu_buffer_rsrc_t R, u32 off) {
     return __builtin_amdgcn_raw_buffer_load_b128(R, off, 0, kDeviceCoherent);
 }
-// the state of three chunks as loaded, and whether all counts are `need`
-__device__ inline bool take_state(Chunk a, Chunk b, Chunk c, u32 need, BodyState& s) {
-    s.v = {__uint_as_float(a.x), __uint_as_float(a.z), __uint_as_float(b.x)};
-    s.w = {__uint_as_float(b.z), __uint_as_float(c.x), __uint_as_float(c.z)};
-    return a.y == need && a.w == need && b.y == need && b.w == need && c.y == need && c.w == need;
-}
-__device__ inline void publish_state(__amdgpu_buffer_rsrc_t R, u32 body, u32 count, const V& v, const V& w) {
-    const u32 off = body * kStateBytes;
-    const Chunk a = {__float_as_uint(v.x), count, __float_as_uint(v.y), count};
-    const Chunk b = {__float_as_uint(v.z), count, __float_as_uint(w.x), count};
-    const Chunk c = {__float_as_uint(w.y), count, __float_as_uint(w.z), count};
+__device__ inline void store_chunk(__amdgpu_buffer_rsrc_t R, u32 off, float lin, float ang, u32 count) {
+    const Chunk a = {__float_as_uint(lin), count, __float_as_uint(ang), count};
     __builtin_amdgcn_raw_buffer_store_b128(a, R, off, 0, kDeviceCoherent);
-    __builtin_amdgcn_raw_buffer_store_b128(b, R, off + 16u, 0, kDeviceCoherent);
-    __builtin_amdgcn_raw_buffer_store_b128(c, R, off + 32u, 0, kDeviceCoherent);
 }
 // Clock cycles before a body still (need - seen) updates short of a
 // waiting manager is polled again: about one solve hop per missing update
@@ -1251,124 +1258,73 @@ __device__ inline u64 poll_delay(u32 need, u32 seen) {
     return d <= 1u ? 0ull : static_cast<u64>(min(d - 1u, 32u)) * kPollHopCycles;
 }
 
-// One manager's rows of one iteration (scene.cpp:8853-9148). info: (body0,
-// body1, manager) of a partition-sorted position. Rows and patches are read
-// with plain loads: the same thread solves the same manager in every
-// iteration, and nothing else writes them during the sweep.
-// s0 / s1: the bodies' states as taken by the sweep (zero for a static
-// side); ima / imb: inverse masses. The updated states are published with
-// counts c0 / c1; fin0 / fin1: the body's last update of the sweep, whose
-// state also goes to the plain rows read after the sweep.
-// Loads the contact and friction rows in use (row counts come with the
-// position record), all at once.
-__device__ inline void load_rows(const Ws& W, int4 info, CRow (&rows)[4], FRow (&frows)[4]) {
-    const u32 m = static_cast<u32>(info.z);
-    const u32 no = static_cast<u32>(info.w) & 0xffu;
-    const u32 anchors = (static_cast<u32>(info.w) >> 8) & 0xffu;
-#pragma unroll
-    for (u32 q = 0; q < 4; ++q) {
-        if (q < no) rows[q] = W.crow[4 * m + q];
-        if (q < 2 * anchors) frows[q] = W.frow[4 * m + q];
-    }
+// The eight lanes of one manager. Every exchange is a DPP move inside them:
+// a quad broadcast (one lane's value to the four of its side) or the
+// half-row mirror, which hands each lane a value of the other side (the
+// values exchanged are the same in all four lanes of a side). The eight
+// lanes always run together, so a DPP source is never an inactive lane.
+constexpr int kDppMirror8 = 0x141;  // row_half_mirror
+template <int CTRL>
+__device__ inline float dpp(float x) {
+    return __uint_as_float(
+        static_cast<u32>(__builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(x)), CTRL, 0xf, 0xf, true)));
 }
-// rows / frows: the manager's rows as loaded by load_rows.
-__device__ void solve_manager(const Ws& W, int4 info, CRow (&rows)[4], FRow (&frows)[4], float4 fric, const BodyState& s0,
-                              const BodyState& s1, float ima, float imb, u32 c0, u32 c1, bool snap0, bool snap1,
-                              bool fin0, bool fin1, u32 iter, u32 pos_iters, u32 total_iters) {
-    const int i0 = info.x, i1 = info.y;
-    const u32 m = static_cast<u32>(info.z);
-    const u32 no = static_cast<u32>(info.w) & 0xffu;
-    const u32 anchors = (static_cast<u32>(info.w) >> 8) & 0xffu;
-    V va = s0.v, vb = s1.v, wa = s0.w, wb = s1.w;
-    bool bad = false;
-    float normal_impulse = 0.0f;
-#pragma unroll
-    for (u32 q = 0; q < 4; ++q) {
-        if (q >= no) break;
-        CRow& r = rows[q];
-        const V n{r.nx, r.ny, r.nz};
-        const V ra{r.rax, r.ray, r.raz}, rb{r.rbx, r.rby, r.rbz};
-        const float nv = vdot(n, va) - vdot(n, vb) + vdot(wa, ra) - vdot(wb, rb);
-        const float err = iter < pos_iters ? r.biased : r.unbiased;
-        const float x = -nv * r.vm + err;
-        const float dc = smax(x, -r.applied);
-        const float next = smin(r.max_impulse, 1.0f * r.applied + dc);
-        if (W.tape && iter < W.tape_iters)
-            W.tape_c[static_cast<std::size_t>(iter) * 4 * W.nm + 4 * m + q] =
-                r.max_impulse < 1.0f * r.applied + dc ? 2 : (x < -r.applied ? 0 : 1);
-        const float delta = next - r.applied;
-        const float da = delta * ima;
-        const float db = delta * imb;
-        va = {va.x + n.x * da, va.y + n.y * da, va.z + n.z * da};
-        vb = {vb.x - n.x * db, vb.y - n.y * db, vb.z - n.z * db};
-        wa = {wa.x + ra.x * delta, wa.y + ra.y * delta, wa.z + ra.z * delta};
-        wb = {wb.x - rb.x * delta, wb.y - rb.y * delta, wb.z - rb.z * delta};
-        r.applied = next;
-        W.crow[4 * m + q].applied = next;
-        normal_impulse += next;
-    }
-    if (W.tape && iter < W.tape_iters) W.tape_ni[static_cast<std::size_t>(iter) * W.nm + m] = normal_impulse;
-    if ((iter >= pos_iters || pos_iters - iter <= 3u) && anchors) {
-        const float coef = anchors == 2 ? 0.5f : 1.0f;
-        const float max_static = fric.x * coef * normal_impulse;
-        const float max_dynamic = fric.y * coef * normal_impulse;
-        bool broken = false;
-#pragma unroll
-        for (u32 k = 0; k < 4; ++k) {
-            if (k >= anchors * 2) break;
-            FRow& fr = frows[k];
-            const V t{fr.tx, fr.ty, fr.tz};
-            const V ra{fr.rax, fr.ray, fr.raz}, rb{fr.rbx, fr.rby, fr.rbz};
-            const float td = vdot(t, va) - vdot(t, vb) + vdot(wa, ra) - vdot(wb, rb);
-            const float bias = iter < pos_iters ? fr.bias : 0.0f;
-            const float cand = fr.applied + (fr.target - bias - td) * fr.vm;
-            const bool clamped = fabsf(cand) > max_static;
-            const float next = clamped ? smin(max_dynamic, smax(-max_dynamic, cand)) : cand;
-            if (W.tape && iter < W.tape_iters)
-                W.tape_f[static_cast<std::size_t>(iter) * 4 * W.nm + 4 * m + k] =
-                    !clamped ? 0 : (max_dynamic < cand ? 2 : (cand < -max_dynamic ? 3 : 1));
-            const float delta = next - fr.applied;
-            const float da = delta * ima;
-            const float db = delta * imb;
-            va = {va.x + t.x * da, va.y + t.y * da, va.z + t.z * da};
-            vb = {vb.x - t.x * db, vb.y - t.y * db, vb.z - t.z * db};
-            wa = {wa.x + ra.x * delta, wa.y + ra.y * delta, wa.z + ra.z * delta};
-            wb = {wb.x - rb.x * delta, wb.y - rb.y * delta, wb.z - rb.z * delta};
-            fr.applied = next;
-            W.frow[4 * m + k].applied = next;
-            broken |= clamped;
-        }
-        if (iter + 1 == total_iters) W.patches[m].flags = (__float_as_uint(fric.z) & ~1u) | (broken ? 1u : 0u);
-    }
-    // a velocity component once non-finite stays so through later row
-    // updates (sums with finite or non-finite terms), so the final check
-    // equals a check after every row
-    bad = !finite3(va) || !finite3(vb) || !finite3(wa) || !finite3(wb);
-    if (bad) raise_flag(W, FYZZ_DY_NONFINITE);
-    if (i0 >= 0) {
-        publish_state(state_rsrc(W), static_cast<u32>(i0), c0, va, wa);
-        const float4 l = make_float4(va.x, va.y, va.z, ima), a = make_float4(wa.x, wa.y, wa.z, 0.f);
-        if (snap0) {
-            W.mlin[i0] = l;
-            W.mang[i0] = a;
-        }
-        if (fin0) {
-            W.lin[i0] = l;
-            W.ang[i0] = a;
-        }
-    }
-    if (i1 >= 0) {
-        publish_state(state_rsrc(W), static_cast<u32>(i1), c1, vb, wb);
-        const float4 l = make_float4(vb.x, vb.y, vb.z, imb), a = make_float4(wb.x, wb.y, wb.z, 0.f);
-        if (snap1) {
-            W.mlin[i1] = l;
-            W.mang[i1] = a;
-        }
-        if (fin1) {
-            W.lin[i1] = l;
-            W.ang[i1] = a;
-        }
-    }
+template <int K>
+__device__ inline float quad(float x) { return dpp<K * 0x55>(x); }
+__device__ inline float other_side(float x) { return dpp<kDppMirror8>(x); }
+// x.x + y.y + z.z of the side's three component products, in that order
+__device__ inline float side_sum(float p) { return (quad<0>(p) + quad<1>(p)) + quad<2>(p); }
+// -x for the second side (adding it is the subtraction, zero signs included)
+__device__ inline float signed_by(float x, u32 flip) { return __uint_as_float(__float_as_uint(x) ^ flip); }
+// Whether `ok` holds in all eight lanes.
+__device__ inline bool octet_all(bool ok) { return ((__ballot(ok) >> (lane_id() & ~7u)) & 0xffull) == 0xffull; }
+
+__device__ inline bool octet_any(bool ok) { return ((__ballot(ok) >> (lane_id() & ~7u)) & 0xffull) != 0ull; }
+
+// A row's values in one lane: its component's direction and lever, and the
+// row's scalars: velocity multiplier, error (contact) or target less bias
+// (friction), maximum impulse.
+struct LaneRow {
+    float d, r, vm, e, top;
+};
+// Both rows of a pair from the lane's float4 of it (see Ws::rows); e:
+// the scalar lanes' error of the iteration.
+__device__ inline void unpack_rows(const float4& x, float e, bool side1, LaneRow& first, LaneRow& second) {
+    first.d = x.x;
+    first.r = x.y;
+    second.d = x.z;
+    second.r = x.w;
+    // the scalar lane (3) of each side, then the other side's
+    const float vm = quad<3>(x.x), er = quad<3>(e), top = quad<3>(x.w);
+    const float ovm = other_side(vm), oer = other_side(er), otop = other_side(top);
+    first.vm = side1 ? ovm : vm;
+    first.e = side1 ? oer : er;
+    first.top = side1 ? otop : top;
+    second.vm = side1 ? vm : ovm;
+    second.e = side1 ? er : oer;
+    second.top = side1 ? top : otop;
+}
+// Applied impulses (lane q holds contact row q or friction row q - 4) of
+// contact row K and friction row K in every lane.
+template <int K>
+__device__ inline void unpack_applied(float x, bool side1, float& contact, float& friction) {
+    const float own = quad<K>(x), oth = other_side(own);
+    contact = side1 ? oth : own;
+    friction = side1 ? own : oth;
+}
+
+// One side's velocity state in its four lanes, and what a row's relative
+// velocity is made of: direction . (side 0) - direction . (side 1) +
+// lever . (side 0) - lever . (side 1), in that order.
+struct LaneState {
+    float v, w;
+};
+__device__ inline float relative(const LaneState& s, float d, float r, bool side1) {
+    const float lin = side_sum(d * s.v), ang = side_sum(s.w * r);
+    const float olin = other_side(lin), oang = other_side(ang);
+    const float l0 = side1 ? olin : lin, l1 = side1 ? lin : olin;
+    const float a0 = side1 ? oang : ang, a1 = side1 ? ang : oang;
+    return l0 - l1 + a0 - a1;
 }
 
 // Position then velocity iterations over the partitions in order, motion
@@ -1378,33 +1334,49 @@ __device__ void solve_manager(const Ws& W, int4 info, CRow (&rows)[4], FRow (&fr
 // the Gauss-Seidel result depends only on each body seeing its managers'
 // updates in that order. A body's state words count the updates applied
 // to it; the manager at rank r among the body's d managers (by partition)
-// runs in iteration t once all six words carry t*d + r, and publishes its
-// result with t*d + r + 1. Thread k solves positions k, k + T, ...
-// in every iteration (T threads), in sequence order, each as soon as it is
-// ready (a lane waits without holding back the rest of its wave). The
-// earliest unsolved (iteration, position) always has its predecessors done
-// and its thread resident (cooperative launch), so the sweep always
-// advances; waits are bounded regardless (a status flag, not a hang).
+// runs in iteration t once all words carry t*d + r, and publishes its
+// result with t*d + r + 1. Eight lanes solve a manager (four per body);
+// octet k solves positions k, k + T, ... in every iteration (T octets), in
+// sequence order, each as soon as it is ready (an octet waits without
+// holding back the rest of its wave). The earliest unsolved (iteration,
+// position) always has its predecessors done and its octet resident
+// (cooperative launch), so the sweep always advances; waits are bounded
+// regardless (a status flag, not a hang).
+//
+// What bounds it: the chain of dependent managers (partitions x iterations
+// hops), each hop a store made visible, a poll that finds it, and the
+// solve. With one thread per manager a wave held up to 64 managers that
+// became ready a few at a time, and each such group cost a full serial
+// solve of both bodies' components; a poll read a body's line in two round
+// trips. Eight lanes read the line in one request, solve the components
+// side by side (about a third of the dependent instructions) and poll for
+// eight managers per wave instead of 64.
 __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
-    const u32 tid = blockIdx.x * kBlock + threadIdx.x;
-    const u32 nthreads = gridDim.x * kBlock;
+    const u32 q = threadIdx.x & 7u, c = q & 3u;
+    const bool side1 = q >= 4u;
+    const u32 flip = side1 ? 0x80000000u : 0u;
+    const u32 slot = (blockIdx.x * kBlock + threadIdx.x) >> 3;
+    const u32 nslots = (gridDim.x * kBlock) >> 3;
     const u32 np = min(ld(&W.ctr[kNParts]), kMaxParts);
     const u32 pos_iters = ld(&W.ctr[kPosIters]);
     const u32 vel_iters = max(ld(&W.ctr[kVelIters]), 1u);
     const u32 total = pos_iters + vel_iters;
     const u32 n = np ? W.part_off[np] : 0u;
-    u32 iter = 0, i = tid, spins = 0, idle = 0;
+    u32 iter = 0, i = slot, spins = 0, idle = 0;
     const __amdgpu_buffer_rsrc_t R = state_rsrc(W);
-    u64 wake0 = 0, wake1 = 0;  // earliest clock at which each body is polled again
-    bool have = false, ready0 = false, ready1 = false;
+    u64 wake = 0;  // earliest clock at which the side's body is polled again
+    bool have = false, ready = false;
     int4 info = make_int4(-1, -1, 0, 0);
     uint4 rk = make_uint4(0u, 0u, 0u, 0u);
-    BodyState s0{}, s1{};
-    float ima = 0.f, imb = 0.f;
-    CRow rows[4];
-    FRow frows[4];
+    int body = -1;
+    u32 need = 0;
+    Chunk st = {0u, 0u, 0u, 0u};
+    float4 x[4] = {};
+    LaneRow row[8] = {};
+    float ap[8] = {};
+    float app = 0.f;
     float4 fric = make_float4(0.f, 0.f, 0.f, 0.f);  // static and dynamic friction, patch flags
-    // the position record of the thread's next position, loaded while the
+    // the position record of the octet's next position, loaded while the
     // current manager waits (positions repeat in every iteration)
     u32 next_pos = kNone;
     int4 next_info = info;
@@ -1413,10 +1385,11 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
         bool progress = false;
         while (iter < total && i >= n) {
             ++iter;
-            i = tid;
+            i = slot;
         }
         if (iter < total) {
-            if (!have) {
+            const bool fresh = !have;
+            if (fresh) {
                 if (next_pos == i) {
                     info = next_info;
                     rk = next_rk;
@@ -1425,76 +1398,141 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
                     rk = W.srank[i];
                 }
                 have = true;
-                ready0 = info.x < 0;
-                ready1 = info.y < 0;
-                wake0 = wake1 = 0;
-                s0 = BodyState{};
-                s1 = BodyState{};
-                // inverse masses: constant through the sweep
-                ima = info.x >= 0 ? W.lin[info.x].w : 0.f;
-                imb = info.y >= 0 ? W.lin[info.y].w : 0.f;
-                // the rows are loaded while the bodies are awaited (only
-                // this thread writes them during the sweep)
-                load_rows(W, info, rows, frows);
-                {
-                    // the patch's friction coefficients and flags (only
-                    // this thread writes them during the sweep)
-                    const fyzz_dy_patch& P = W.patches[info.z];
-                    fric = make_float4(P.static_friction, P.dynamic_friction, __uint_as_float(P.flags), 0.f);
-                }
-                const u32 nx = i + nthreads < n ? i + nthreads : tid;
+                body = side1 ? info.y : info.x;
+                need = side1 ? iter * rk.w + rk.y : iter * rk.z + rk.x;
+                ready = body < 0;
+                wake = 0;
+                st = Chunk{0u, 0u, 0u, 0u};
+                // the rows are loaded while the bodies are awaited; only
+                // this octet writes the applied impulses during the sweep,
+                // each lane its own
+                const float4* rows = W.rows + static_cast<std::size_t>(kRowQuads) * i + q;
+                const u32 no = static_cast<u32>(info.w) & 0xffu, anchors = (static_cast<u32>(info.w) >> 8) & 0xffu;
+                x[0] = rows[0];
+                if (no > 2u) x[1] = rows[kRowLanes];
+                if (anchors) x[2] = rows[2 * kRowLanes];
+                if (anchors > 1u) x[3] = rows[3 * kRowLanes];
+                app = W.app[8ull * i + q];
+                fric = W.fric[i];
+                const u32 nx = i + nslots < n ? i + nslots : slot;
                 if (nx < n) {
                     next_pos = nx;
                     next_info = W.sinfo[nx];
                     next_rk = W.srank[nx];
                 }
             }
-            // a body whose count reached the awaited value stays there
+            // A body whose count reached the awaited value stays there
             // until this manager runs: its state is kept, not polled again.
             // A body still `need - seen` updates short is polled again only
             // after about that many solve hops: waiting lanes would
             // otherwise keep the memory system busy with polls that cannot
             // succeed, slowing the hops they wait for.
-            const u32 need0 = iter * rk.z + rk.x, need1 = iter * rk.w + rk.y;
             const u64 now = clock64();
-            // both bodies' first chunks in flight together, then the other
-            // chunks of the bodies whose first chunk carries the awaited
-            // count (the count it carries: the updates the body has had)
-            const bool p0 = !ready0 && now >= wake0, p1 = !ready1 && now >= wake1;
-            const bool polled = p0 || p1;
-            const u32 o0 = static_cast<u32>(info.x) * kStateBytes, o1 = static_cast<u32>(info.y) * kStateBytes;
-            Chunk a0, b0, c0, a1, b1, c1;
-            if (p0) a0 = load_chunk(R, o0);
-            if (p1) a1 = load_chunk(R, o1);
-            const bool m0 = p0 && a0.y == need0, m1 = p1 && a1.y == need1;
-            if (m0) {
-                b0 = load_chunk(R, o0 + 16u);
-                c0 = load_chunk(R, o0 + 32u);
+            const bool poll = !ready && now >= wake;
+            if (poll) {
+                st = load_chunk(R, static_cast<u32>(body) * kStateBytes + 16u * c);
+                const bool got = st.y == need && st.w == need;
+                ready = ((__ballot(got) >> (lane_id() & ~3u)) & 0xfull) == 0xfull;
+                // (the first lane's count for all four)
+                const u32 seen = __float_as_uint(quad<0>(__uint_as_float(st.y)));
+                if (!ready) wake = now + poll_delay(need, seen);
             }
-            if (m1) {
-                b1 = load_chunk(R, o1 + 16u);
-                c1 = load_chunk(R, o1 + 32u);
+            if (fresh) {
+                // off the dependency chain: the wait for the poll covers the
+                // row loads issued before it
+                const bool pos = iter < pos_iters;
+                unpack_rows(x[0], pos ? x[0].y : x[0].z, side1, row[0], row[1]);
+                unpack_rows(x[1], pos ? x[1].y : x[1].z, side1, row[2], row[3]);
+                unpack_rows(x[2], x[2].z - (pos ? x[2].y : 0.0f), side1, row[4], row[5]);
+                unpack_rows(x[3], x[3].z - (pos ? x[3].y : 0.0f), side1, row[6], row[7]);
+                unpack_applied<0>(app, side1, ap[0], ap[4]);
+                unpack_applied<1>(app, side1, ap[1], ap[5]);
+                unpack_applied<2>(app, side1, ap[2], ap[6]);
+                unpack_applied<3>(app, side1, ap[3], ap[7]);
             }
-            if (p0) {
-                ready0 = m0 && take_state(a0, b0, c0, need0, s0);
-                if (!ready0) wake0 = now + poll_delay(need0, a0.y);
-            }
-            if (p1) {
-                ready1 = m1 && take_state(a1, b1, c1, need1, s1);
-                if (!ready1) wake1 = now + poll_delay(need1, a1.y);
-            }
-            if (ready0 && ready1) {
-                const bool snap = iter + 1 == pos_iters, last = iter + 1 == total;
-                const bool end0 = rk.x + 1 == rk.z, end1 = rk.y + 1 == rk.w;
-                solve_manager(W, info, rows, frows, fric, s0, s1, ima, imb, need0 + 1u, need1 + 1u, snap && end0,
-                              snap && end1, last && end0, last && end1, iter, pos_iters, total);
+            if (octet_all(ready)) {
+                const u32 no = static_cast<u32>(info.w) & 0xffu, anchors = (static_cast<u32>(info.w) >> 8) & 0xffu;
+                LaneState s{__uint_as_float(st.x), __uint_as_float(st.z)};
+                const float im = quad<3>(s.v);
+                u32 branch = 0;  // tape: the branch of the lane's row
+                float normal_impulse = 0.0f;
+#pragma unroll
+                for (u32 k = 0; k < 4; ++k) {
+                    if (k >= no) break;
+                    const LaneRow& r = row[k];
+                    const float nv = relative(s, r.d, r.r, side1);
+                    const float xx = -nv * r.vm + r.e;
+                    const float dc = smax(xx, -ap[k]);
+                    const float sum = 1.0f * ap[k] + dc;
+                    const float next = smin(r.top, sum);
+                    if (q == k) branch = r.top < sum ? 2u : (xx < -ap[k] ? 0u : 1u);
+                    const float delta = next - ap[k];
+                    const float dm = delta * im;
+                    s.v += signed_by(r.d * dm, flip);
+                    s.w += signed_by(r.r * delta, flip);
+                    if (q == k) app = next;
+                    normal_impulse += next;
+                }
+                const u32 m = static_cast<u32>(info.z);
+                const bool rub = (iter >= pos_iters || pos_iters - iter <= 3u) && anchors;
+                if (rub) {
+                    const float coef = anchors == 2 ? 0.5f : 1.0f;
+                    const float max_static = fric.x * coef * normal_impulse;
+                    const float max_dynamic = fric.y * coef * normal_impulse;
+                    bool broken = false;
+#pragma unroll
+                    for (u32 k = 0; k < 4; ++k) {
+                        if (k >= anchors * 2) break;
+                        const LaneRow& r = row[4 + k];
+                        const float td = relative(s, r.d, r.r, side1);
+                        const float cand = ap[4 + k] + (r.e - td) * r.vm;
+                        const bool clamped = fabsf(cand) > max_static;
+                        const float next = clamped ? smin(max_dynamic, smax(-max_dynamic, cand)) : cand;
+                        if (q == 4 + k) branch = !clamped ? 0u : (max_dynamic < cand ? 2u : (cand < -max_dynamic ? 3u : 1u));
+                        const float delta = next - ap[4 + k];
+                        const float dm = delta * im;
+                        s.v += signed_by(r.d * dm, flip);
+                        s.w += signed_by(r.r * delta, flip);
+                        if (q == 4 + k) app = next;
+                        broken |= clamped;
+                    }
+                    if (iter + 1 == total && q == 0)
+                        W.patches[m].flags = (__float_as_uint(fric.z) & ~1u) | (broken ? 1u : 0u);
+                }
+                if (c == 3u) s = LaneState{im, 0.0f};
+                if (body >= 0) store_chunk(R, static_cast<u32>(body) * kStateBytes + 16u * c, s.v, s.w, need + 1u);
+                // a velocity component once non-finite stays so through
+                // later row updates (sums with finite or non-finite terms),
+                // so the final check equals a check after every row
+                if (c < 3u && (!isfinite(s.v) || !isfinite(s.w))) raise_flag(W, FYZZ_DY_NONFINITE);
+                W.app[8ull * i + q] = app;
+                const bool end = side1 ? rk.y + 1 == rk.w : rk.x + 1 == rk.z;
+                if (body >= 0 && end) {
+                    if (iter + 1 == pos_iters) {
+                        reinterpret_cast<float*>(W.mlin + body)[c] = s.v;
+                        reinterpret_cast<float*>(W.mang + body)[c] = s.w;
+                    }
+                    if (iter + 1 == total) {
+                        reinterpret_cast<float*>(W.lin + body)[c] = s.v;
+                        reinterpret_cast<float*>(W.ang + body)[c] = s.w;
+                    }
+                }
+                if (W.tape && iter < W.tape_iters) {
+                    const std::size_t t = static_cast<std::size_t>(iter) * 4 * W.nm + 4 * m + c;
+                    if (!side1) {
+                        if (c < no) W.tape_c[t] = static_cast<uint8_t>(branch);
+                    } else if (rub && c < 2 * anchors) {
+                        W.tape_f[t] = static_cast<uint8_t>(branch);
+                    }
+                    if (q == 0) W.tape_ni[static_cast<std::size_t>(iter) * W.nm + m] = normal_impulse;
+                }
                 have = false;
-                i += nthreads;
+                i += nslots;
                 progress = true;
-                spins = 0;  // the budget bounds one wait, not the thread's whole sweep
-            } else if (polled && ++spins > kSpinLimit) {
+                spins = 0;  // the budget bounds one wait, not the octet's whole sweep
+            } else if (octet_any(poll) && ++spins > kSpinLimit) {
                 raise_flag(W, FYZZ_DY_LOGIC);
-                iter = total;  // give up on this thread's work
+                iter = total;  // give up on this octet's work
             }
         }
         if (!__ballot(iter < total)) break;
@@ -1538,7 +1576,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_init(Ws W) {
     if (t < nm) W.a_df[t] = 0.f;
 }
 
-__device__ void adjoint_manager(const Ws& W, u32 m, u32 iter, u32 pos_iters) {
+__device__ void adjoint_manager(const Ws& W, u32 pos, u32 iter, u32 pos_iters) {
+    const u32 m = W.sorted[pos];
     const fyzz_dy_manager& M = W.mg[m];
     const int i0 = M.body0, i1 = M.body1;
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1555,9 +1594,8 @@ __device__ void adjoint_manager(const Ws& W, u32 m, u32 iter, u32 pos_iters) {
         const float df = P.dynamic_friction;
         float a_maxd = 0.0f;
         for (int k = static_cast<int>(anchors * 2) - 1; k >= 0; --k) {
-            const FRow& fr = W.frow[4 * m + k];
-            const V t{fr.tx, fr.ty, fr.tz};
-            const V ra{fr.rax, fr.ray, fr.raz}, rb{fr.rbx, fr.rby, fr.rbz};
+            const RowOut fr = read_row(W, pos, 4 + k);
+            const V t = fr.d, ra = fr.ra, rb = fr.rb;
             const float a_delta = vdot(t, ava) * ima - vdot(t, avb) * imb + vdot(ra, awa) - vdot(rb, awb);
             const float a_next = W.a_fapp[4 * m + k] + a_delta;
             float a_applied = -a_delta;
@@ -1570,8 +1608,8 @@ __device__ void adjoint_manager(const Ws& W, u32 m, u32 iter, u32 pos_iters) {
             else
                 a_maxd -= a_next;
             a_applied += a_cand;
-            W.a_tgt[4 * m + k] += fr.vm * a_cand;
-            const float a_td = -fr.vm * a_cand;
+            W.a_tgt[4 * m + k] += fr.s.x * a_cand;
+            const float a_td = -fr.s.x * a_cand;
             ava = vadd(ava, vmul(t, a_td));
             avb = vsub(avb, vmul(t, a_td));
             awa = vadd(awa, vmul(ra, a_td));
@@ -1584,15 +1622,14 @@ __device__ void adjoint_manager(const Ws& W, u32 m, u32 iter, u32 pos_iters) {
     }
     const u32 no = W.order[m] & 0xffu;
     for (int q = static_cast<int>(no) - 1; q >= 0; --q) {
-        const CRow& r = W.crow[4 * m + q];
-        const V n{r.nx, r.ny, r.nz};
-        const V ra{r.rax, r.ray, r.raz}, rb{r.rbx, r.rby, r.rbz};
+        const RowOut r = read_row(W, pos, q);
+        const V n = r.d, ra = r.ra, rb = r.rb;
         const float a_delta = vdot(n, ava) * ima - vdot(n, avb) * imb + vdot(ra, awa) - vdot(rb, awb);
         const float a_next = W.a_capp[4 * m + q] + a_delta + a_ni;
         float a_applied = -a_delta;
         if (W.tape_c[row_base + q] == 1) {
             a_applied += a_next;
-            const float a_nv = -r.vm * a_next;
+            const float a_nv = -r.s.x * a_next;
             W.a_err[4 * m + q] += a_next;
             ava = vadd(ava, vmul(n, a_nv));
             avb = vsub(avb, vmul(n, a_nv));
@@ -1642,7 +1679,7 @@ __global__ __launch_bounds__(kBlock) void k_pgs_adjoint(Ws W) {
         }
         for (u32 p = np; p-- > 0;) {
             const u32 lo = W.part_off[p], hi = W.part_off[p + 1];
-            for (u32 i = lo + tid; i < hi; i += nthreads) adjoint_manager(W, W.sorted[i], it, pos_iters);
+            for (u32 i = lo + tid; i < hi; i += nthreads) adjoint_manager(W, i, it, pos_iters);
             grid_sync(W, gen);
         }
     }
@@ -1655,13 +1692,14 @@ __global__ __launch_bounds__(kBlock) void k_adj_rows(Ws W) {
     if (m >= mcount(W) || W.part[m] >= kMaxParts) return;
     const fyzz_dy_manager& M = W.mg[m];
     const int i0 = M.body0, i1 = M.body1;
+    const u32 pos = W.pos_of[m];
     V ava{0.f, 0.f, 0.f}, avb{0.f, 0.f, 0.f}, awa{0.f, 0.f, 0.f}, awb{0.f, 0.f, 0.f};
     const u32 no = W.order[m] & 0xffu;
     for (u32 q = 0; q < no; ++q) {
-        const CRow& r = W.crow[4 * m + q];
+        const RowOut r = read_row(W, pos, q);
         const float4 x0 = W.craw[2 * (4 * m + q)], x1 = W.craw[2 * (4 * m + q) + 1];
-        const float a_vrel = x0.w * r.vm * W.a_err[4 * m + q];
-        const V n{r.nx, r.ny, r.nz};
+        const float a_vrel = x0.w * r.s.x * W.a_err[4 * m + q];
+        const V n = r.d;
         ava = vadd(ava, vmul(n, a_vrel));
         avb = vsub(avb, vmul(n, a_vrel));
         awa = vadd(awa, vmul(f3(x0), a_vrel));
@@ -1669,9 +1707,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_rows(Ws W) {
     }
     const fyzz_dy_patch& P = W.patches[m];
     for (u32 k = 0; k < 2 * P.anchor_count; ++k) {
-        const FRow& fr = W.frow[4 * m + k];
+        const V t = read_row(W, pos, 4 + k).d;
         const float a_t = W.a_tgt[4 * m + k];
-        const V t{fr.tx, fr.ty, fr.tz};
         // target = -(t . (va - vb) + (ra x t) . wa - (rb x t) . wb)
         ava = vsub(ava, vmul(t, a_t));
         avb = vadd(avb, vmul(t, a_t));
@@ -1913,11 +1950,13 @@ __global__ __launch_bounds__(kBlock) void k_outputs(Ws W) {
         if (W.with_rows && W.part[m] < kMaxParts) {
             const u32 o = W.order[m];
             const u32 no = min(o & 0xffu, 4u);
+            const float4 app = *reinterpret_cast<const float4*>(W.app + 8ull * W.pos_of[m]);
+            const float applied[4] = {app.x, app.y, app.z, app.w};
 #pragma unroll
             for (u32 q = 0; q < 4; ++q) {
                 if (q >= no) continue;
                 const u32 slot = (o >> (8 + 4 * q)) & 0xfu;
-                const float v = W.crow[4 * m + q].applied;
+                const float v = applied[q];
 #pragma unroll
                 for (u32 k = 0; k < 4; ++k) out[k] = slot == k ? v : out[k];
             }
@@ -1967,11 +2006,12 @@ __global__ __launch_bounds__(kBlock) void k_anchors(Ws W, fyzz_friction_anchors*
             r.position[k][0] = cp.x + rot.x;
             r.position[k][1] = cp.y + rot.y;
             r.position[k][2] = cp.z + rot.z;
-            const FRow& x = W.frow[4 * m + 2 * k];
-            const FRow& y = W.frow[4 * m + 2 * k + 1];
-            r.impulse[k][0] = static_cast<double>(x.tx) * x.applied + static_cast<double>(y.tx) * y.applied;
-            r.impulse[k][1] = static_cast<double>(x.ty) * x.applied + static_cast<double>(y.ty) * y.applied;
-            r.impulse[k][2] = static_cast<double>(x.tz) * x.applied + static_cast<double>(y.tz) * y.applied;
+            const u32 pos = W.pos_of[m];
+            const V x = read_row(W, pos, 4 + 2 * k).d, y = read_row(W, pos, 5 + 2 * k).d;
+            const float ax = W.app[8ull * pos + 4 + 2 * k], ay = W.app[8ull * pos + 5 + 2 * k];
+            r.impulse[k][0] = static_cast<double>(x.x) * ax + static_cast<double>(y.x) * ay;
+            r.impulse[k][1] = static_cast<double>(x.y) * ax + static_cast<double>(y.y) * ay;
+            r.impulse[k][2] = static_cast<double>(x.z) * ax + static_cast<double>(y.z) * ay;
         }
     }
     out[m] = r;
@@ -1995,8 +2035,8 @@ struct fyzz_hip_dy {
     DevBuf<uint4> srank;
     DevBuf<u32> erank, pos_of;
     DevBuf<u64> vst;
-    DevBuf<dy::CRow> crow;
-    DevBuf<dy::FRow> frow;
+    DevBuf<float4> rows, fric;
+    DevBuf<float> app;
     DevBuf<u32> part_count, part_off, part_fill, blocksums, ctr, flags, bar;
     // tape mode
     bool tape = false;
@@ -2248,8 +2288,9 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         d->pos_of.reserve(nm);
         for (auto* b : {&d->part, &d->pend, &d->sorted, &d->order}) b->reserve(nm);
         d->dd.reserve(nm);
-        d->crow.reserve(4 * nm);
-        d->frow.reserve(4 * nm);
+        d->rows.reserve(dy::kRowQuads * nm);
+        d->app.reserve(8 * nm);
+        d->fric.reserve(nm);
         d->part_count.reserve(dy::kMaxParts + 1);
         d->part_off.reserve(dy::kMaxParts + 1);
         d->part_fill.reserve(dy::kMaxParts);
@@ -2296,8 +2337,9 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         w.sorted = d->sorted.get();
         w.order = d->order.get();
         w.dd = d->dd.get();
-        w.crow = d->crow.get();
-        w.frow = d->frow.get();
+        w.rows = d->rows.get();
+        w.app = d->app.get();
+        w.fric = d->fric.get();
         w.part_count = d->part_count.get();
         w.part_off = d->part_off.get();
         w.part_fill = d->part_fill.get();
@@ -2308,8 +2350,8 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         // every workspace array the step kernels touch must exist
         const void* need[] = {w.pv, w.pw, w.lin, w.ang, w.mlin, w.mang, w.rpos, w.rq, w.sii, w.has_row,
                               w.deg, w.off, w.fill, w.max_dyn, w.body_mask, w.inc, w.pred, w.part, w.pend,
-                              w.sorted, w.order, w.entry, w.sinfo, w.srank, w.erank, w.vst, w.pos_of, w.crow,
-                              w.frow,
+                              w.sorted, w.order, w.entry, w.sinfo, w.srank, w.erank, w.vst, w.pos_of, w.rows,
+                              w.app, w.fric,
                               w.part_count, w.part_off, w.part_fill, w.blocksums, w.ctr, w.flags, w.bar};
         for (const void* q : need) FYZZ_REQUIRE(q != nullptr, kDeviceError, "dy_create: workspace array missing");
         *out = d.release();
