@@ -49,7 +49,7 @@ constexpr u32 kMaxParts = 4096;       // partitions per step
 constexpr u32 kMaxPending = 65536;    // managers left for overflow waves
 constexpr int kBlock = 256;
 constexpr int kCoopBlocks = 64;       // workgroups of the cooperative launches
-constexpr int kPgsBlocks = 256;       // workgroups of the sweep (no grid barrier there)
+constexpr int kPgsBlocks = 512;       // workgroups of the sweep (see k_pgs)
 
 // device counters
 enum : u32 { kFront0 = 0, kFront1, kFront2, kPend, kNParts, kPosIters, kVelIters, kRounds, kContacts, kFrictionRows,
@@ -62,7 +62,8 @@ enum : u32 { kFront0 = 0, kFront1, kFront2, kPend, kNParts, kPosIters, kVelIters
 // c = q & 3) of pair p holds
 //   c < 3: (direction_c, lever_c) of the pair's first row, then of its
 //          second (direction: contact normal or tangent; lever: the side's
-//          angular part of the row)
+//          angular part of the row), negated for side 1, whose terms enter
+//          a row's relative velocity and its own update with a minus
 //   c = 3: the scalars of the first row (side 0) or the second (side 1):
 //          contact (velocity multiplier, biased error, unbiased error,
 //          maximum impulse), friction (velocity multiplier, bias, target, 0)
@@ -847,9 +848,9 @@ __device__ inline void store_rows(float4* o, const RowOut& x, const RowOut& y) {
     o[1] = make_float4(x.d.y, x.ra.y, y.d.y, y.ra.y);
     o[2] = make_float4(x.d.z, x.ra.z, y.d.z, y.ra.z);
     o[3] = x.s;
-    o[4] = make_float4(x.d.x, x.rb.x, y.d.x, y.rb.x);
-    o[5] = make_float4(x.d.y, x.rb.y, y.d.y, y.rb.y);
-    o[6] = make_float4(x.d.z, x.rb.z, y.d.z, y.rb.z);
+    o[4] = make_float4(-x.d.x, -x.rb.x, -y.d.x, -y.rb.x);
+    o[5] = make_float4(-x.d.y, -x.rb.y, -y.d.y, -y.rb.y);
+    o[6] = make_float4(-x.d.z, -x.rb.z, -y.d.z, -y.rb.z);
     o[7] = y.s;
 }
 // Row r (0-3 contact, 4-7 friction) of a position, read back by one thread.
@@ -860,7 +861,7 @@ __device__ inline RowOut read_row(const Ws& W, u32 pos, u32 r) {
     const float4 x = o[0], y = o[1], z = o[2], bx = o[4], by = o[5], bz = o[6];
     v.d = second ? V{x.z, y.z, z.z} : V{x.x, y.x, z.x};
     v.ra = second ? V{x.w, y.w, z.w} : V{x.y, y.y, z.y};
-    v.rb = second ? V{bx.w, by.w, bz.w} : V{bx.y, by.y, bz.y};
+    v.rb = second ? V{-bx.w, -by.w, -bz.w} : V{-bx.y, -by.y, -bz.y};
     v.s = o[second ? 7 : 3];
     return v;
 }
@@ -1272,14 +1273,25 @@ __device__ inline float dpp(float x) {
 template <int K>
 __device__ inline float quad(float x) { return dpp<K * 0x55>(x); }
 __device__ inline float other_side(float x) { return dpp<kDppMirror8>(x); }
-// x.x + y.y + z.z of the side's three component products, in that order
-__device__ inline float side_sum(float p) { return (quad<0>(p) + quad<1>(p)) + quad<2>(p); }
-// -x for the second side (adding it is the subtraction, zero signs included)
-__device__ inline float signed_by(float x, u32 flip) { return __uint_as_float(__float_as_uint(x) ^ flip); }
-// Whether `ok` holds in all eight lanes.
-__device__ inline bool octet_all(bool ok) { return ((__ballot(ok) >> (lane_id() & ~7u)) & 0xffull) == 0xffull; }
+// A value of side 0 (the same in its four lanes), or of side 1, in all
+// eight lanes: the mirror into the other side's quads only (the bank mask
+// names a row's quads), the side's own quads keep theirs.
+template <int BANKS>
+__device__ inline float mirror_into(float x) {
+    const int v = static_cast<int>(__float_as_uint(x));
+    return __uint_as_float(static_cast<u32>(__builtin_amdgcn_update_dpp(v, v, kDppMirror8, 0xf, BANKS, false)));
+}
+__device__ inline float of_side0(float x) { return mirror_into<0xa>(x); }
+__device__ inline float of_side1(float x) { return mirror_into<0x5>(x); }
 
-__device__ inline bool octet_any(bool ok) { return ((__ballot(ok) >> (lane_id() & ~7u)) & 0xffull) != 0ull; }
+// The bits set in any of the four lanes of a side, and of either side
+// (values equal in the four lanes).
+template <int CTRL>
+__device__ inline u32 dpp_or(u32 x) {
+    return x | static_cast<u32>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, 0xf, 0xf, true));
+}
+__device__ inline u32 quad_or(u32 x) { return dpp_or<0x4e>(dpp_or<0xb1>(x)); }  // lane ^ 1, then lane ^ 2
+__device__ inline u32 sides_or(u32 x) { return dpp_or<kDppMirror8>(x); }
 
 // A row's values in one lane: its component's direction and lever, and the
 // row's scalars: velocity multiplier, error (contact) or target less bias
@@ -1289,42 +1301,46 @@ struct LaneRow {
 };
 // Both rows of a pair from the lane's float4 of it (see Ws::rows); e:
 // the scalar lanes' error of the iteration.
-__device__ inline void unpack_rows(const float4& x, float e, bool side1, LaneRow& first, LaneRow& second) {
+__device__ inline void unpack_rows(const float4& x, float e, LaneRow& first, LaneRow& second) {
     first.d = x.x;
     first.r = x.y;
     second.d = x.z;
     second.r = x.w;
-    // the scalar lane (3) of each side, then the other side's
+    // the scalar lane (3) of each side: the first row's is side 0's
     const float vm = quad<3>(x.x), er = quad<3>(e), top = quad<3>(x.w);
-    const float ovm = other_side(vm), oer = other_side(er), otop = other_side(top);
-    first.vm = side1 ? ovm : vm;
-    first.e = side1 ? oer : er;
-    first.top = side1 ? otop : top;
-    second.vm = side1 ? vm : ovm;
-    second.e = side1 ? er : oer;
-    second.top = side1 ? top : otop;
+    first.vm = of_side0(vm);
+    first.e = of_side0(er);
+    first.top = of_side0(top);
+    second.vm = of_side1(vm);
+    second.e = of_side1(er);
+    second.top = of_side1(top);
 }
 // Applied impulses (lane q holds contact row q or friction row q - 4) of
 // contact row K and friction row K in every lane.
 template <int K>
-__device__ inline void unpack_applied(float x, bool side1, float& contact, float& friction) {
-    const float own = quad<K>(x), oth = other_side(own);
-    contact = side1 ? oth : own;
-    friction = side1 ? own : oth;
+__device__ inline void unpack_applied(float x, float& contact, float& friction) {
+    const float own = quad<K>(x);
+    contact = of_side0(own);
+    friction = of_side1(own);
 }
 
-// One side's velocity state in its four lanes, and what a row's relative
-// velocity is made of: direction . (side 0) - direction . (side 1) +
-// lever . (side 0) - lever . (side 1), in that order.
+// One side's velocity state in its four lanes, and a row's relative
+// velocity: direction . (side 0) - direction . (side 1) + lever . (side 0) -
+// lever . (side 1), in that order. Side 1 holds its row negated, so its
+// terms come with their minus: each product is the exact negative, and so
+// is each sum but for the sign of a zero. That sign reaches nothing: the
+// relative velocity is only subtracted from an error, scaled and added to
+// an applied impulse, which is never -0 (it starts at +0, and a sum is -0
+// only of two -0).
 struct LaneState {
     float v, w;
 };
-__device__ inline float relative(const LaneState& s, float d, float r, bool side1) {
-    const float lin = side_sum(d * s.v), ang = side_sum(s.w * r);
-    const float olin = other_side(lin), oang = other_side(ang);
-    const float l0 = side1 ? olin : lin, l1 = side1 ? lin : olin;
-    const float a0 = side1 ? oang : ang, a1 = side1 ? ang : oang;
-    return l0 - l1 + a0 - a1;
+__device__ inline float relative(const LaneState& s, float d, float r) {
+    const float pv = d * s.v, pw = s.w * r;
+    const float v0 = quad<0>(pv), w0 = quad<0>(pw);
+    const float v1 = v0 + quad<1>(pv), w1 = w0 + quad<1>(pw);
+    const float lin = v1 + quad<2>(pv), ang = w1 + quad<2>(pw);
+    return ((lin + other_side(lin)) + of_side0(ang)) + of_side1(ang);
 }
 
 // Position then velocity iterations over the partitions in order, motion
@@ -1347,14 +1363,24 @@ __device__ inline float relative(const LaneState& s, float d, float r, bool side
 // hops), each hop a store made visible, a poll that finds it, and the
 // solve. With one thread per manager a wave held up to 64 managers that
 // became ready a few at a time, and each such group cost a full serial
-// solve of both bodies' components; a poll read a body's line in two round
-// trips. Eight lanes read the line in one request, solve the components
-// side by side (about a third of the dependent instructions) and poll for
-// eight managers per wave instead of 64.
+// solve of both bodies' components (1.8 us); a poll read a body's line in
+// two round trips. Eight lanes read the line in one request, solve the
+// components side by side and poll for eight managers per wave instead of
+// 64. Measured in steps (us per sweep, one thread per manager before): the
+// formed pile of 100,000 boxes (230k managers, 19 partitions) 580 -> 317,
+// a heap of 3,001 (800 managers, 10 partitions) 229 -> 120, 2,048 scenes
+// 146 -> 99. By solve-time stamps on the heap a hop is 1.7 us: 0.7 us of
+// solve (0.45 without friction rows), the rest visibility and polls.
+// Variants that lost: the next position's rows loaded one position ahead
+// (pile 407 -> 437), the solve issued between the polls and their answers
+// (341 -> 505). 512 workgroups: pile 382 at 256, 317 at 512, 317 at 768;
+// the scenes 91 at 256, 106 at 768.
+// kTape: also records each row's branch for the adjoint (a variant of its
+// own, so that a plain sweep carries none of it).
+template <bool kTape>
 __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
     const u32 q = threadIdx.x & 7u, c = q & 3u;
     const bool side1 = q >= 4u;
-    const u32 flip = side1 ? 0x80000000u : 0u;
     const u32 slot = (blockIdx.x * kBlock + threadIdx.x) >> 3;
     const u32 nslots = (gridDim.x * kBlock) >> 3;
     const u32 np = min(ld(&W.ctr[kNParts]), kMaxParts);
@@ -1365,7 +1391,9 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
     u32 iter = 0, i = slot, spins = 0, idle = 0;
     const __amdgpu_buffer_rsrc_t R = state_rsrc(W);
     u64 wake = 0;  // earliest clock at which the side's body is polled again
-    bool have = false, ready = false;
+    u64 now = 0;   // the clock as of the last pass (its read overlaps that pass's polls)
+    bool have = false;
+    u32 miss = 0;  // zero once the side's body state is taken (or the side is static)
     int4 info = make_int4(-1, -1, 0, 0);
     uint4 rk = make_uint4(0u, 0u, 0u, 0u);
     int body = -1;
@@ -1400,22 +1428,23 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
                 have = true;
                 body = side1 ? info.y : info.x;
                 need = side1 ? iter * rk.w + rk.y : iter * rk.z + rk.x;
-                ready = body < 0;
+                miss = body < 0 ? 0u : 1u;
                 wake = 0;
                 st = Chunk{0u, 0u, 0u, 0u};
                 // the rows are loaded while the bodies are awaited; only
                 // this octet writes the applied impulses during the sweep,
-                // each lane its own
-                const float4* rows = W.rows + static_cast<std::size_t>(kRowQuads) * i + q;
-                const u32 no = static_cast<u32>(info.w) & 0xffu, anchors = (static_cast<u32>(info.w) >> 8) & 0xffu;
-                x[0] = rows[0];
-                if (no > 2u) x[1] = rows[kRowLanes];
-                if (anchors) x[2] = rows[2 * kRowLanes];
-                if (anchors > 1u) x[3] = rows[3 * kRowLanes];
-                app = W.app[8ull * i + q];
-                fric = W.fric[i];
-                const u32 nx = i + nslots < n ? i + nslots : slot;
-                if (nx < n) {
+                // each lane its own. An octet with a single position keeps
+                // its rows and impulses in the lanes.
+                if (iter == 0 || n > nslots) {
+                    const float4* rows = W.rows + static_cast<std::size_t>(kRowQuads) * i + q;
+                    const u32 no = static_cast<u32>(info.w) & 0xffu, anchors = (static_cast<u32>(info.w) >> 8) & 0xffu;
+                    x[0] = rows[0];
+                    if (no > 2u) x[1] = rows[kRowLanes];
+                    if (anchors) x[2] = rows[2 * kRowLanes];
+                    if (anchors > 1u) x[3] = rows[3 * kRowLanes];
+                    app = W.app[8ull * i + q];
+                    fric = W.fric[i];
+                    const u32 nx = i + nslots < n ? i + nslots : slot;
                     next_pos = nx;
                     next_info = W.sinfo[nx];
                     next_rk = W.srank[nx];
@@ -1427,50 +1456,55 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
             // after about that many solve hops: waiting lanes would
             // otherwise keep the memory system busy with polls that cannot
             // succeed, slowing the hops they wait for.
-            const u64 now = clock64();
-            const bool poll = !ready && now >= wake;
+            const bool poll = miss && now >= wake;
             if (poll) {
                 st = load_chunk(R, static_cast<u32>(body) * kStateBytes + 16u * c);
-                const bool got = st.y == need && st.w == need;
-                ready = ((__ballot(got) >> (lane_id() & ~3u)) & 0xfull) == 0xfull;
+                miss = quad_or((st.y ^ need) | (st.w ^ need));
                 // (the first lane's count for all four)
                 const u32 seen = __float_as_uint(quad<0>(__uint_as_float(st.y)));
-                if (!ready) wake = now + poll_delay(need, seen);
+                if (miss) wake = now + poll_delay(need, seen);
             }
             if (fresh) {
                 // off the dependency chain: the wait for the poll covers the
                 // row loads issued before it
                 const bool pos = iter < pos_iters;
-                unpack_rows(x[0], pos ? x[0].y : x[0].z, side1, row[0], row[1]);
-                unpack_rows(x[1], pos ? x[1].y : x[1].z, side1, row[2], row[3]);
-                unpack_rows(x[2], x[2].z - (pos ? x[2].y : 0.0f), side1, row[4], row[5]);
-                unpack_rows(x[3], x[3].z - (pos ? x[3].y : 0.0f), side1, row[6], row[7]);
-                unpack_applied<0>(app, side1, ap[0], ap[4]);
-                unpack_applied<1>(app, side1, ap[1], ap[5]);
-                unpack_applied<2>(app, side1, ap[2], ap[6]);
-                unpack_applied<3>(app, side1, ap[3], ap[7]);
+                unpack_rows(x[0], pos ? x[0].y : x[0].z, row[0], row[1]);
+                unpack_rows(x[1], pos ? x[1].y : x[1].z, row[2], row[3]);
+                unpack_rows(x[2], x[2].z - (pos ? x[2].y : 0.0f), row[4], row[5]);
+                unpack_rows(x[3], x[3].z - (pos ? x[3].y : 0.0f), row[6], row[7]);
+                unpack_applied<0>(app, ap[0], ap[4]);
+                unpack_applied<1>(app, ap[1], ap[5]);
+                unpack_applied<2>(app, ap[2], ap[6]);
+                unpack_applied<3>(app, ap[3], ap[7]);
             }
-            if (octet_all(ready)) {
+            if (!sides_or(miss)) {
                 const u32 no = static_cast<u32>(info.w) & 0xffu, anchors = (static_cast<u32>(info.w) >> 8) & 0xffu;
                 LaneState s{__uint_as_float(st.x), __uint_as_float(st.z)};
                 const float im = quad<3>(s.v);
-                u32 branch = 0;  // tape: the branch of the lane's row
+                [[maybe_unused]] u32 branch = 0;  // tape: the branch of the lane's row
                 float normal_impulse = 0.0f;
 #pragma unroll
                 for (u32 k = 0; k < 4; ++k) {
                     if (k >= no) break;
                     const LaneRow& r = row[k];
-                    const float nv = relative(s, r.d, r.r, side1);
+                    const float nv = relative(s, r.d, r.r);
                     const float xx = -nv * r.vm + r.e;
-                    const float dc = smax(xx, -ap[k]);
-                    const float sum = 1.0f * ap[k] + dc;
-                    const float next = smin(r.top, sum);
-                    if (q == k) branch = r.top < sum ? 2u : (xx < -ap[k] ? 0u : 1u);
+                    // max and min as the hardware has them: the operands
+                    // differ or are the same bits (an applied impulse is
+                    // never -0, so xx and -ap[k] are no mixed zeros), and a
+                    // NaN stays in the velocities and is flagged below
+                    const float dc = fmaxf(xx, -ap[k]);
+                    const float sum = ap[k] + dc;
+                    const float next = fminf(r.top, sum);
+                    if constexpr (kTape) {
+                        const u32 br = r.top < sum ? 2u : (xx < -ap[k] ? 0u : 1u);
+                        branch = q == k ? br : branch;
+                    }
                     const float delta = next - ap[k];
                     const float dm = delta * im;
-                    s.v += signed_by(r.d * dm, flip);
-                    s.w += signed_by(r.r * delta, flip);
-                    if (q == k) app = next;
+                    s.v += r.d * dm;
+                    s.w += r.r * delta;
+                    app = q == k ? next : app;
                     normal_impulse += next;
                 }
                 const u32 m = static_cast<u32>(info.z);
@@ -1479,21 +1513,29 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
                     const float coef = anchors == 2 ? 0.5f : 1.0f;
                     const float max_static = fric.x * coef * normal_impulse;
                     const float max_dynamic = fric.y * coef * normal_impulse;
+                    const float min_dynamic = 0.0f - max_dynamic;
                     bool broken = false;
 #pragma unroll
                     for (u32 k = 0; k < 4; ++k) {
                         if (k >= anchors * 2) break;
                         const LaneRow& r = row[4 + k];
-                        const float td = relative(s, r.d, r.r, side1);
+                        const float td = relative(s, r.d, r.r);
                         const float cand = ap[4 + k] + (r.e - td) * r.vm;
                         const bool clamped = fabsf(cand) > max_static;
-                        const float next = clamped ? smin(max_dynamic, smax(-max_dynamic, cand)) : cand;
-                        if (q == 4 + k) branch = !clamped ? 0u : (max_dynamic < cand ? 2u : (cand < -max_dynamic ? 3u : 1u));
+                        // a clamped candidate lies beyond +-max_static,
+                        // which is at least max_dynamic: its clamp is the
+                        // bound of its sign (+0 when the bound is 0)
+                        const float bound = cand > 0.0f ? max_dynamic : min_dynamic;
+                        const float next = clamped ? bound : cand;
+                        if constexpr (kTape) {
+                            const u32 br = !clamped ? 0u : (max_dynamic < cand ? 2u : (cand < -max_dynamic ? 3u : 1u));
+                            branch = q == 4 + k ? br : branch;
+                        }
                         const float delta = next - ap[4 + k];
                         const float dm = delta * im;
-                        s.v += signed_by(r.d * dm, flip);
-                        s.w += signed_by(r.r * delta, flip);
-                        if (q == 4 + k) app = next;
+                        s.v += r.d * dm;
+                        s.w += r.r * delta;
+                        app = q == 4 + k ? next : app;
                         broken |= clamped;
                     }
                     if (iter + 1 == total && q == 0)
@@ -1505,7 +1547,7 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
                 // later row updates (sums with finite or non-finite terms),
                 // so the final check equals a check after every row
                 if (c < 3u && (!isfinite(s.v) || !isfinite(s.w))) raise_flag(W, FYZZ_DY_NONFINITE);
-                W.app[8ull * i + q] = app;
+                if (iter + 1 == total || n > nslots) W.app[8ull * i + q] = app;
                 const bool end = side1 ? rk.y + 1 == rk.w : rk.x + 1 == rk.z;
                 if (body >= 0 && end) {
                     if (iter + 1 == pos_iters) {
@@ -1517,7 +1559,7 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
                         reinterpret_cast<float*>(W.ang + body)[c] = s.w;
                     }
                 }
-                if (W.tape && iter < W.tape_iters) {
+                if (kTape && iter < W.tape_iters) {
                     const std::size_t t = static_cast<std::size_t>(iter) * 4 * W.nm + 4 * m + c;
                     if (!side1) {
                         if (c < no) W.tape_c[t] = static_cast<uint8_t>(branch);
@@ -1530,7 +1572,7 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
                 i += nslots;
                 progress = true;
                 spins = 0;  // the budget bounds one wait, not the octet's whole sweep
-            } else if (octet_any(poll) && ++spins > kSpinLimit) {
+            } else if (sides_or(poll ? 1u : 0u) && ++spins > kSpinLimit) {
                 raise_flag(W, FYZZ_DY_LOGIC);
                 iter = total;  // give up on this octet's work
             }
@@ -1538,7 +1580,12 @@ __global__ __launch_bounds__(kBlock) void k_pgs(Ws W) {
         if (!__ballot(iter < total)) break;
         idle = __ballot(progress) ? 0u : idle + 1u;
         wait_backoff(idle);
+        now = clock64();
     }
+}
+
+inline const void* pgs_kernel(bool tape) {
+    return tape ? reinterpret_cast<const void*>(&k_pgs<true>) : reinterpret_cast<const void*>(&k_pgs<false>);
 }
 
 // --------------------------------------------------------------- adjoint
@@ -2149,7 +2196,7 @@ void dy_solve(fyzz_hip_dy* d) {
     d->taped_step = d->ws.tape != 0;
     if (!d->ws.nm) return;
     ProfScope ps(&d->ctx->prof, "dy.pgs", d->ctx->stream);
-    launch_coop(reinterpret_cast<const void*>(&dy::k_pgs), d->coop_blocks_pgs, d->ws, d->ctx->stream,
+    launch_coop(dy::pgs_kernel(d->ws.tape != 0), d->coop_blocks_pgs, d->ws, d->ctx->stream,
                 d->plain_launch || !d->ctx->cooperative);
 }
 
@@ -2233,7 +2280,7 @@ void set_plain_launch(fyzz_hip_dy* d, bool plain) { d->plain_launch = plain; }
 void set_coop_blocks(fyzz_hip_dy* d, int partition_blocks, int pgs_blocks) {
     const int cap_p = coop_blocks(reinterpret_cast<const void*>(&k_part_color), d->ctx->device, 1 << 30);
     // the sweep has no grid barrier: its cap is the resident capacity
-    const int cap_s = resident_blocks(reinterpret_cast<const void*>(&k_pgs), d->ctx->device);
+    const int cap_s = resident_blocks(pgs_kernel(true), d->ctx->device);
     FYZZ_REQUIRE(partition_blocks > 0 && pgs_blocks > 0, kInvalidArgument, "dy: workgroup counts must be positive");
     d->coop_blocks_partition = std::min(partition_blocks, cap_p);
     d->coop_blocks_pgs = std::min(pgs_blocks, cap_s);
@@ -2243,9 +2290,9 @@ void set_coop_blocks(fyzz_hip_dy* d, int partition_blocks, int pgs_blocks) {
 }
 void effective_blocks(int device, int partition_blocks, int pgs_blocks, int* partition_out, int* pgs_out) {
     const void* color = reinterpret_cast<const void*>(&k_part_color);
-    const void* pgs = reinterpret_cast<const void*>(&k_pgs);
+    const void* pgs = pgs_kernel(true);
     *partition_out = partition_blocks > 0 ? coop_blocks(color, device, partition_blocks) : coop_blocks(color, device, 128);
-    *pgs_out = pgs_blocks > 0 ? std::min(pgs_blocks, resident_blocks(pgs, device)) : coop_blocks(pgs, device, kPgsBlocks);
+    *pgs_out = pgs_blocks > 0 ? std::min(pgs_blocks, resident_blocks(pgs, device)) : std::min(resident_blocks(pgs, device), kPgsBlocks);
 }
 void coop_blocks_of(fyzz_hip_dy* d, int* partition_blocks, int* pgs_blocks) {
     *partition_blocks = d->coop_blocks_partition;
@@ -2300,7 +2347,7 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         FYZZ_HIP_CHECK(hipMemset(d->bar.get(), 0, dy::kBarWords * sizeof(u32)));
         // 128 colouring workgroups measured best on the pile (64: +7 us, 256: +2 us)
         d->coop_blocks_partition = coop_blocks(reinterpret_cast<const void*>(&dy::k_part_color), ctx->device, 128);
-        d->coop_blocks_pgs = coop_blocks(reinterpret_cast<const void*>(&dy::k_pgs), ctx->device, dy::kPgsBlocks);
+        d->coop_blocks_pgs = std::min(resident_blocks(dy::pgs_kernel(true), ctx->device), dy::kPgsBlocks);
         // the reverse sweep keeps grid barriers between partitions
         d->coop_blocks_adjoint = coop_blocks(reinterpret_cast<const void*>(&dy::k_pgs_adjoint), ctx->device);
         // room for the largest grid the autotuner may pick, and for the
