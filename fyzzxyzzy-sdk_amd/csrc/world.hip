@@ -1085,7 +1085,9 @@ struct fyzz_hip_world {
     hipStream_t gstream = nullptr;
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     float gdt[2] = {0.0f, 0.0f};
-    hipEvent_t gev_in = nullptr, gev_out = nullptr;
+    hipEvent_t gev_out = nullptr;
+    hipStream_t glast = nullptr;  // the stream of the last graph step (gev_out follows it there)
+    bool glaunched = false;
     // independent scenes (per-scene broadphase instead of one SAP)
     std::vector<u32> scene_counts;
     u32 n_scenes = 0;
@@ -1122,7 +1124,6 @@ struct fyzz_hip_world {
         if (order_auth) fyzz_hip_islands_destroy(order_auth);
         for (auto& g : gexec)
             if (g) (void)hipGraphExecDestroy(g);
-        if (gev_in) (void)hipEventDestroy(gev_in);
         if (gev_out) (void)hipEventDestroy(gev_out);
         if (gstream) (void)hipStreamDestroy(gstream);
         if (dy) fyzz_hip_dy_destroy(dy);
@@ -1790,9 +1791,11 @@ void step(fyzz_hip_world* w, float dt) {
 // One step through a captured graph. The step's host-side toggles (pair
 // list, caches, friction history) flip every step, so a graph per parity
 // is captured on first use (or when dt changes) and replayed afterwards;
-// the history stamps come from the device step counter. The graphs run on
-// the world's own stream, ordered after and before the context stream's
-// work by events.
+// the history stamps come from the device step counter. A step is captured
+// on a stream of the world's own and launched on the context's: launched on
+// the world's own stream, ordered by two events, a step moved between
+// hardware queues twice (a 64-box world 757 us per step against 345, the
+// formed pile of 100,000 boxes 2,930 against 2,300).
 void step_graph(fyzz_hip_world* w, float dt) {
     if (!w->uploaded) upload(w);
     if (!w->n) {
@@ -1808,13 +1811,10 @@ void step_graph(fyzz_hip_world* w, float dt) {
     }
     if (!w->gstream) {
         FYZZ_HIP_CHECK(hipStreamCreateWithFlags(&w->gstream, hipStreamNonBlocking));
-        FYZZ_HIP_CHECK(hipEventCreateWithFlags(&w->gev_in, hipEventDisableTiming));
         FYZZ_HIP_CHECK(hipEventCreateWithFlags(&w->gev_out, hipEventDisableTiming));
     }
     const int parity = static_cast<int>(w->step_index & 1u);
     hipStream_t outer = w->ctx->stream;
-    FYZZ_HIP_CHECK(hipEventRecord(w->gev_in, outer));
-    FYZZ_HIP_CHECK(hipStreamWaitEvent(w->gstream, w->gev_in, 0));
     if (!w->gexec[parity] || w->gdt[parity] != dt) {
         if (w->gexec[parity]) {
             FYZZ_HIP_CHECK(hipGraphExecDestroy(w->gexec[parity]));
@@ -1854,9 +1854,12 @@ void step_graph(fyzz_hip_world* w, float dt) {
         w->scur ^= 1;
         if (!w->n_scenes) sap::replay_advance(w->sap);
     }
-    FYZZ_HIP_CHECK(hipGraphLaunch(w->gexec[parity], w->gstream));
-    FYZZ_HIP_CHECK(hipEventRecord(w->gev_out, w->gstream));
-    FYZZ_HIP_CHECK(hipStreamWaitEvent(outer, w->gev_out, 0));
+    // steps stay in order when the context has moved to another stream
+    if (w->glaunched && w->glast != outer) FYZZ_HIP_CHECK(hipStreamWaitEvent(outer, w->gev_out, 0));
+    FYZZ_HIP_CHECK(hipGraphLaunch(w->gexec[parity], outer));
+    FYZZ_HIP_CHECK(hipEventRecord(w->gev_out, outer));
+    w->glast = outer;
+    w->glaunched = true;
 }
 
 // The pair list the next step starts from (the last step's current list).

@@ -177,6 +177,34 @@ def test_graph_steps_match_eager_steps_sap_world(torch_cuda):
         cb.close()
 
 
+def test_graph_steps_stay_in_order_across_streams(torch_cuda):
+    """Graph steps launched on the context's stream, which changes every
+    three steps with no synchronization between, against eager steps: the
+    steps stay in order and the states are bit-identical."""
+    from fyzz_amd import Context
+    from fyzz_amd._lib import lib
+    torch = torch_cuda
+    sc = small_pile(6)
+    ca, cb = Context(0), Context(0)
+    wa, wb = make_world(ca, sc), make_world(cb, sc)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    handles = [None] + [s.cuda_stream for s in streams]
+    try:
+        for s in range(36):
+            wa.step(1 / 120)
+            if s % 3 == 0:
+                assert lib().fyzz_hip_set_stream(cb.h, handles[(s // 3) % 3]) == 0
+            wb.step_graph(1 / 120)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(wb.body_states(), wa.body_states())
+        assert wb.stats() == wa.stats()
+    finally:
+        wa.close()
+        wb.close()
+        ca.close()
+        cb.close()
+
+
 def _free_boxes(seed=scenes.SEED_BASE + 41, side=20, spacing=3.0):
     """side x side boxes (half extents U[0.2, 0.6] m) on a grid 3 m apart,
     0.6-2.0 m above the floor, with seeded yaw and small velocities: they
