@@ -125,9 +125,10 @@ struct Ws {
     float* adj_v_in;
     float* adj_w_in;
     float* adj_friction;  // per body: d loss / d dynamic friction
-    float4 *a_lin, *a_ang;
     float4* a_side;  // [4 nm] per manager and side: (velocity adjoint, friction adjoint), (angular adjoint, 0)
-    float *a_capp, *a_fapp, *a_err, *a_tgt, *a_df;
+    // by position: the applied impulses' adjoint, the errors' (contact) and targets' (friction), as app
+    float *a_app, *a_acc;
+    float* a_df;  // per manager: the dynamic friction's
 };
 
 __device__ inline u32 ld(const u32* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -1343,6 +1344,17 @@ __device__ inline float relative(const LaneState& s, float d, float r) {
     return ((lin + other_side(lin)) + of_side0(ang)) + of_side1(ang);
 }
 
+// The reverse of a row's velocity update: (direction . side 0) im0 -
+// (direction . side 1) im1 + lever . (side 0) - lever . (side 1), in that
+// order (signs as in relative).
+__device__ inline float reverse_relative(const LaneState& s, float d, float r, float im) {
+    const float pv = d * s.v, pw = r * s.w;
+    const float v0 = quad<0>(pv), w0 = quad<0>(pw);
+    const float v1 = v0 + quad<1>(pv), w1 = w0 + quad<1>(pw);
+    const float lin = (v1 + quad<2>(pv)) * im, ang = w1 + quad<2>(pw);
+    return ((lin + other_side(lin)) + of_side0(ang)) + of_side1(ang);
+}
+
 // Position then velocity iterations over the partitions in order, motion
 // snapshotted after the last position iteration (scene.cpp:9136-9146),
 // without grid barriers. The sweep is the sequence (iteration, sorted
@@ -1601,134 +1613,198 @@ inline const void* pgs_kernel(bool tape) {
 
 __device__ inline V ld3(const float* p, u32 i) { return {p[3 * i], p[3 * i + 1], p[3 * i + 2]}; }
 
-// adjoint state at the end of the sweeps
+// adjoint state at the end of the sweeps, in the state lines (no updates
+// yet; the inverse mass as in the sweep)
 __global__ __launch_bounds__(kBlock) void k_adj_init(Ws W) {
     const u32 t = blockIdx.x * kBlock + threadIdx.x;
     if (t < W.nb) {
         const V av = ld3(W.adj_v_out, t), aw = ld3(W.adj_w_out, t);
         const float4 c0 = W.sii[3 * t], c1 = W.sii[3 * t + 1], c2 = W.sii[3 * t + 2];
         // v_out = v_pre + lin; w_out = w_pre + S ang (S symmetric)
-        W.a_lin[t] = make_float4(av.x, av.y, av.z, 0.f);
-        W.a_ang[t] = make_float4(c0.x * aw.x + c0.y * aw.y + c0.z * aw.z, c1.x * aw.x + c1.y * aw.y + c1.z * aw.z,
-                                 c2.x * aw.x + c2.y * aw.y + c2.z * aw.z, 0.f);
+        const float lin[4] = {av.x, av.y, av.z, W.lin[t].w};
+        const float ang[4] = {c0.x * aw.x + c0.y * aw.y + c0.z * aw.z, c1.x * aw.x + c1.y * aw.y + c1.z * aw.z,
+                              c2.x * aw.x + c2.y * aw.y + c2.z * aw.z, 0.f};
+        for (u32 k = 0; k < 4; ++k) {
+            W.vst[8 * t + 2 * k] = __float_as_uint(lin[k]);
+            W.vst[8 * t + 2 * k + 1] = __float_as_uint(ang[k]);
+        }
         W.adj_friction[t] = 0.0f;
     }
     const u32 nm = mcount(W);
-    if (t < 4 * nm) {
-        W.a_capp[t] = 0.f;
-        W.a_fapp[t] = 0.f;
-        W.a_err[t] = 0.f;
-        W.a_tgt[t] = 0.f;
+    if (t < 8 * nm) {
+        W.a_app[t] = 0.f;
+        W.a_acc[t] = 0.f;
     }
     if (t < nm) W.a_df[t] = 0.f;
-}
-
-__device__ void adjoint_manager(const Ws& W, u32 pos, u32 iter, u32 pos_iters) {
-    const u32 m = W.sorted[pos];
-    const fyzz_dy_manager& M = W.mg[m];
-    const int i0 = M.body0, i1 = M.body1;
-    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    const float ima = i0 >= 0 ? W.lin[i0].w : 0.f, imb = i1 >= 0 ? W.lin[i1].w : 0.f;
-    V ava = f3(i0 >= 0 ? W.a_lin[i0] : z4), avb = f3(i1 >= 0 ? W.a_lin[i1] : z4);
-    V awa = f3(i0 >= 0 ? W.a_ang[i0] : z4), awb = f3(i1 >= 0 ? W.a_ang[i1] : z4);
-    const fyzz_dy_patch& P = W.patches[m];
-    const u32 anchors = P.anchor_count;
-    const std::size_t row_base = static_cast<std::size_t>(iter) * 4 * W.nm + 4 * m;
-    float a_ni = 0.0f;
-    if ((iter >= pos_iters || pos_iters - iter <= 3u) && anchors) {
-        const float coef = anchors == 2 ? 0.5f : 1.0f;
-        const float ni = W.tape_ni[static_cast<std::size_t>(iter) * W.nm + m];
-        const float df = P.dynamic_friction;
-        float a_maxd = 0.0f;
-        for (int k = static_cast<int>(anchors * 2) - 1; k >= 0; --k) {
-            const RowOut fr = read_row(W, pos, 4 + k);
-            const V t = fr.d, ra = fr.ra, rb = fr.rb;
-            const float a_delta = vdot(t, ava) * ima - vdot(t, avb) * imb + vdot(ra, awa) - vdot(rb, awb);
-            const float a_next = W.a_fapp[4 * m + k] + a_delta;
-            float a_applied = -a_delta;
-            const uint8_t br = W.tape_f[row_base + k];
-            float a_cand = 0.0f;
-            if (br <= 1)
-                a_cand = a_next;
-            else if (br == 2)
-                a_maxd += a_next;
-            else
-                a_maxd -= a_next;
-            a_applied += a_cand;
-            W.a_tgt[4 * m + k] += fr.s.x * a_cand;
-            const float a_td = -fr.s.x * a_cand;
-            ava = vadd(ava, vmul(t, a_td));
-            avb = vsub(avb, vmul(t, a_td));
-            awa = vadd(awa, vmul(ra, a_td));
-            awb = vsub(awb, vmul(rb, a_td));
-            W.a_fapp[4 * m + k] = a_applied;
-        }
-        // max_dynamic = df * coef * ni
-        W.a_df[m] += coef * ni * a_maxd;
-        a_ni = df * coef * a_maxd;
-    }
-    const u32 no = W.order[m] & 0xffu;
-    for (int q = static_cast<int>(no) - 1; q >= 0; --q) {
-        const RowOut r = read_row(W, pos, q);
-        const V n = r.d, ra = r.ra, rb = r.rb;
-        const float a_delta = vdot(n, ava) * ima - vdot(n, avb) * imb + vdot(ra, awa) - vdot(rb, awb);
-        const float a_next = W.a_capp[4 * m + q] + a_delta + a_ni;
-        float a_applied = -a_delta;
-        if (W.tape_c[row_base + q] == 1) {
-            a_applied += a_next;
-            const float a_nv = -r.s.x * a_next;
-            W.a_err[4 * m + q] += a_next;
-            ava = vadd(ava, vmul(n, a_nv));
-            avb = vsub(avb, vmul(n, a_nv));
-            awa = vadd(awa, vmul(ra, a_nv));
-            awb = vsub(awb, vmul(rb, a_nv));
-        }
-        W.a_capp[4 * m + q] = a_applied;
-    }
-    if (i0 >= 0) {
-        W.a_lin[i0] = make_float4(ava.x, ava.y, ava.z, 0.f);
-        W.a_ang[i0] = make_float4(awa.x, awa.y, awa.z, 0.f);
-    }
-    if (i1 >= 0) {
-        W.a_lin[i1] = make_float4(avb.x, avb.y, avb.z, 0.f);
-        W.a_ang[i1] = make_float4(awb.x, awb.y, awb.z, 0.f);
-    }
 }
 
 // The sweeps in reverse: iterations and partitions backwards. The motion
 // snapshot taken after the last position iteration feeds the position
 // update, so its adjoint (dt x adjoint of the position) joins the
-// velocity-delta adjoint when the reverse reaches that point.
+// velocity-delta adjoint when the reverse reaches that point: the body's
+// first manager of the iteration in reverse order adds it to the state it
+// takes. Dataflow and lanes as in k_pgs, with the order reversed: the
+// manager ranked r of d takes its body's state after (total - 1 - t)*d +
+// d - 1 - r updates. A grid barrier between partitions took 1,535 us per
+// step of 1,024 stacks of 64 boxes and 439 us of 5 stacks; this form takes
+// 231 and 121 us.
 __global__ __launch_bounds__(kBlock) void k_pgs_adjoint(Ws W) {
-    u32 gen = barrier_start(W);
-    const u32 tid = blockIdx.x * kBlock + threadIdx.x;
-    const u32 nthreads = gridDim.x * kBlock;
-    const u32 np = ld(&W.ctr[kNParts]);
+    const u32 q = threadIdx.x & 7u, c = q & 3u;
+    const bool side1 = q >= 4u;
+    const u32 slot = (blockIdx.x * kBlock + threadIdx.x) >> 3;
+    const u32 nslots = (gridDim.x * kBlock) >> 3;
+    const u32 np = min(ld(&W.ctr[kNParts]), kMaxParts);
     const u32 pos_iters = ld(&W.ctr[kPosIters]);
     const u32 vel_iters = max(ld(&W.ctr[kVelIters]), 1u);
     const u32 total = pos_iters + vel_iters;
     if (total > W.tape_iters) {  // the tape does not hold every iteration
-        if (tid == 0) raise_flag(W, FYZZ_DY_OVERFLOW);
+        if (slot == 0 && q == 0) raise_flag(W, FYZZ_DY_OVERFLOW);
         return;
     }
-    for (u32 it = total; it-- > 0;) {
-        if (it + 1 == pos_iters) {
-            for (u32 i = tid; i < W.nb; i += nthreads)
-                if (W.has_row[i]) {
-                    const V ap = ld3(W.adj_p_out, i);
-                    float4 a = W.a_lin[i];
-                    a.x += W.dt * ap.x;
-                    a.y += W.dt * ap.y;
-                    a.z += W.dt * ap.z;
-                    W.a_lin[i] = a;
+    const u32 n = np ? W.part_off[np] : 0u;
+    // `step` counts the reversed iterations; j the reversed positions
+    u32 step = slot < n ? 0u : total, j = slot, spins = 0, idle = 0;
+    const __amdgpu_buffer_rsrc_t R = state_rsrc(W);
+    bool have = false;
+    u32 miss = 0, need = 0;
+    u64 wake = 0, now = 0;  // as in k_pgs
+    int4 info = make_int4(-1, -1, 0, 0);
+    int body = -1;
+    Chunk st = {0u, 0u, 0u, 0u};
+    float4 x[4] = {};
+    LaneRow row[8] = {};
+    float app = 0.f, acc = 0.f, inject = 0.f, ni = 0.f;
+    u32 branch = 0;
+    u32 anchors = 0;  // the patch's anchors and dynamic friction
+    float df = 0.f;
+    while (__ballot(step < total)) {
+        bool progress = false;
+        if (step < total) {
+            const u32 i = n - 1u - j, iter = total - 1u - step;
+            const bool fresh = !have;
+            if (fresh) {
+                info = W.sinfo[i];
+                const uint4 rk = W.srank[i];
+                have = true;
+                body = side1 ? info.y : info.x;
+                const u32 deg = side1 ? rk.w : rk.z, back = deg - 1u - (side1 ? rk.y : rk.x);
+                need = step * deg + back;
+                miss = body < 0 ? 0u : 1u;
+                wake = 0;
+                st = Chunk{0u, 0u, 0u, 0u};
+                const float4* rows = W.rows + static_cast<std::size_t>(kRowQuads) * i + q;
+                const fyzz_dy_patch& P = W.patches[static_cast<u32>(info.z)];
+                anchors = min(P.anchor_count, 2u);
+                df = P.dynamic_friction;
+                const u32 no = static_cast<u32>(info.w) & 0xffu;
+                x[0] = rows[0];
+                if (no > 2u) x[1] = rows[kRowLanes];
+                if (anchors) x[2] = rows[2 * kRowLanes];
+                if (anchors > 1u) x[3] = rows[3 * kRowLanes];
+                app = W.a_app[8ull * i + q];
+                acc = W.a_acc[8ull * i + q];
+                const std::size_t m = static_cast<u32>(info.z), base = static_cast<std::size_t>(iter) * W.nm;
+                branch = (side1 ? W.tape_f : W.tape_c)[4 * (base + m) + c];
+                ni = W.tape_ni[base + m];
+                inject = 0.f;
+                if (iter + 1 == pos_iters && back == 0u && body >= 0 && c < 3u && W.has_row[body])
+                    inject = W.dt * W.adj_p_out[3 * body + c];
+            }
+            const bool poll = miss && now >= wake;
+            if (poll) {
+                st = load_chunk(R, static_cast<u32>(body) * kStateBytes + 16u * c);
+                miss = quad_or((st.y ^ need) | (st.w ^ need));
+                const u32 seen = __float_as_uint(quad<0>(__uint_as_float(st.y)));
+                if (miss) wake = now + poll_delay(need, seen);
+            }
+            if (fresh) {
+                unpack_rows(x[0], 0.f, row[0], row[1]);
+                unpack_rows(x[1], 0.f, row[2], row[3]);
+                unpack_rows(x[2], 0.f, row[4], row[5]);
+                unpack_rows(x[3], 0.f, row[6], row[7]);
+            }
+            if (!sides_or(miss)) {
+                const u32 no = static_cast<u32>(info.w) & 0xffu;
+                LaneState s{__uint_as_float(st.x), __uint_as_float(st.z)};
+                const float im = quad<3>(s.v);
+                if (iter + 1 == pos_iters && c < 3u) s.v += inject;
+                float ap[8];
+                unpack_applied<0>(app, ap[0], ap[4]);
+                unpack_applied<1>(app, ap[1], ap[5]);
+                unpack_applied<2>(app, ap[2], ap[6]);
+                unpack_applied<3>(app, ap[3], ap[7]);
+                // every row's branch in all eight lanes, two bits each
+                u32 br = (branch & 3u) << (2u * q);  // (an unsolved row's byte is unset)
+                br = sides_or(quad_or(br));
+                const u32 m = static_cast<u32>(info.z);
+                float a_ni = 0.0f;
+                if ((iter >= pos_iters || pos_iters - iter <= 3u) && anchors) {
+                    const float coef = anchors == 2 ? 0.5f : 1.0f;
+                    float a_maxd = 0.0f;
+#pragma unroll
+                    for (int k = 3; k >= 0; --k) {
+                        if (k >= static_cast<int>(anchors * 2)) continue;
+                        const LaneRow& r = row[4 + k];
+                        const float a_delta = reverse_relative(s, r.d, r.r, im);
+                        const float a_next = ap[4 + k] + a_delta;
+                        float a_applied = -a_delta;
+                        const u32 b = (br >> (2 * (4 + k))) & 3u;
+                        float a_cand = 0.0f;
+                        if (b <= 1u)
+                            a_cand = a_next;
+                        else if (b == 2u)
+                            a_maxd += a_next;
+                        else
+                            a_maxd -= a_next;
+                        a_applied += a_cand;
+                        const float tgt = acc + r.vm * a_cand;
+                        const float a_td = -r.vm * a_cand;
+                        s.v += r.d * a_td;
+                        s.w += r.r * a_td;
+                        app = q == 4u + k ? a_applied : app;
+                        acc = q == 4u + k ? tgt : acc;
+                    }
+                    // max_dynamic = df * coef * ni
+                    if (q == 0) W.a_df[m] += coef * ni * a_maxd;
+                    a_ni = df * coef * a_maxd;
                 }
-            grid_sync(W, gen);
+#pragma unroll
+                for (int k = 3; k >= 0; --k) {
+                    if (k >= static_cast<int>(no)) continue;
+                    const LaneRow& r = row[k];
+                    const float a_delta = reverse_relative(s, r.d, r.r, im);
+                    const float a_next = ap[k] + a_delta + a_ni;
+                    float a_applied = -a_delta;
+                    if (((br >> (2 * k)) & 3u) == 1u) {
+                        a_applied += a_next;
+                        const float a_nv = -r.vm * a_next;
+                        const float err = acc + a_next;
+                        acc = q == static_cast<u32>(k) ? err : acc;
+                        s.v += r.d * a_nv;
+                        s.w += r.r * a_nv;
+                    }
+                    app = q == static_cast<u32>(k) ? a_applied : app;
+                }
+                if (c == 3u) s = LaneState{im, 0.0f};
+                if (body >= 0) store_chunk(R, static_cast<u32>(body) * kStateBytes + 16u * c, s.v, s.w, need + 1u);
+                W.a_app[8ull * i + q] = app;
+                W.a_acc[8ull * i + q] = acc;
+                have = false;
+                j += nslots;
+                if (j >= n) {
+                    ++step;
+                    j = slot;
+                }
+                progress = true;
+                spins = 0;
+            } else if (sides_or(poll ? 1u : 0u) && ++spins > kSpinLimit) {
+                raise_flag(W, FYZZ_DY_LOGIC);
+                step = total;  // give up on this octet's work
+            }
         }
-        for (u32 p = np; p-- > 0;) {
-            const u32 lo = W.part_off[p], hi = W.part_off[p + 1];
-            for (u32 i = lo + tid; i < hi; i += nthreads) adjoint_manager(W, i, it, pos_iters);
-            grid_sync(W, gen);
-        }
+        idle = __ballot(progress) ? 0u : idle + 1u;
+        wait_backoff(idle);
+        now = clock64();
     }
 }
 
@@ -1745,7 +1821,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_rows(Ws W) {
     for (u32 q = 0; q < no; ++q) {
         const RowOut r = read_row(W, pos, q);
         const float4 x0 = W.craw[2 * (4 * m + q)], x1 = W.craw[2 * (4 * m + q) + 1];
-        const float a_vrel = x0.w * r.s.x * W.a_err[4 * m + q];
+        const float a_vrel = x0.w * r.s.x * W.a_acc[8ull * pos + q];
         const V n = r.d;
         ava = vadd(ava, vmul(n, a_vrel));
         avb = vsub(avb, vmul(n, a_vrel));
@@ -1753,9 +1829,9 @@ __global__ __launch_bounds__(kBlock) void k_adj_rows(Ws W) {
         awb = vsub(awb, vmul(f3(x1), a_vrel));
     }
     const fyzz_dy_patch& P = W.patches[m];
-    for (u32 k = 0; k < 2 * P.anchor_count; ++k) {
+    for (u32 k = 0; k < 2 * min(P.anchor_count, 2u); ++k) {
         const V t = read_row(W, pos, 4 + k).d;
-        const float a_t = W.a_tgt[4 * m + k];
+        const float a_t = W.a_acc[8ull * pos + 4 + k];
         // target = -(t . (va - vb) + (ra x t) . wa - (rb x t) . wb)
         ava = vsub(ava, vmul(t, a_t));
         avb = vadd(avb, vmul(t, a_t));
@@ -2089,8 +2165,8 @@ struct fyzz_hip_dy {
     bool tape = false;
     bool taped_step = false;  // the last solved step recorded a tape
     DevBuf<uint8_t> tape_c, tape_f;
-    DevBuf<float> tape_ni, a_capp, a_fapp, a_err, a_tgt, a_df;
-    DevBuf<float4> craw, fraw, a_lin, a_ang, a_side;
+    DevBuf<float> tape_ni, a_app, a_acc, a_df;
+    DevBuf<float4> craw, fraw, a_side;
     dy::Ws ws{};
     bool prepared = false;
 };
@@ -2221,11 +2297,10 @@ void dy_set_tape(fyzz_hip_dy* d, bool enabled) {
         d->tape_c.reserve(kTapeIters * 4 * nm);
         d->tape_f.reserve(kTapeIters * 4 * nm);
         d->tape_ni.reserve(kTapeIters * nm);
-        for (auto* b : {&d->a_capp, &d->a_fapp, &d->a_err, &d->a_tgt}) b->reserve(4 * nm);
+        for (auto* b : {&d->a_app, &d->a_acc}) b->reserve(8 * nm);
         d->a_df.reserve(nm);
         d->craw.reserve(8 * nm);
         d->fraw.reserve(8 * nm);
-        for (auto* b : {&d->a_lin, &d->a_ang}) b->reserve(nb);
         d->a_side.reserve(4 * nm);
         dy::Ws& w = d->ws;
         w.tape_iters = kTapeIters;
@@ -2234,13 +2309,9 @@ void dy_set_tape(fyzz_hip_dy* d, bool enabled) {
         w.tape_ni = d->tape_ni.p;
         w.craw = d->craw.p;
         w.fraw = d->fraw.p;
-        w.a_capp = d->a_capp.p;
-        w.a_fapp = d->a_fapp.p;
-        w.a_err = d->a_err.p;
-        w.a_tgt = d->a_tgt.p;
+        w.a_app = d->a_app.p;
+        w.a_acc = d->a_acc.p;
         w.a_df = d->a_df.p;
-        w.a_lin = d->a_lin.p;
-        w.a_ang = d->a_ang.p;
         w.a_side = d->a_side.p;
     }
     d->tape = enabled;
@@ -2261,7 +2332,7 @@ void dy_adjoint(fyzz_hip_dy* d, const float* adj_v_out, const float* adj_w_out, 
     w.adj_friction = adj_friction;
     hipStream_t st = d->ctx->stream;
     ProfScope ps(&d->ctx->prof, "dy.adjoint", st);
-    const u32 span = std::max<u32>(w.nb, 4 * w.nm);
+    const u32 span = std::max<u32>(w.nb, 8 * w.nm);
     if (span) hipLaunchKernelGGL(dy::k_adj_init, dim3(grid_for(span, dy::kBlock)), dim3(dy::kBlock), 0, st, w);
     if (w.nm) {
         launch_coop(reinterpret_cast<const void*>(&dy::k_pgs_adjoint), d->coop_blocks_adjoint, w, st,
@@ -2348,8 +2419,8 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         // 128 colouring workgroups measured best on the pile (64: +7 us, 256: +2 us)
         d->coop_blocks_partition = coop_blocks(reinterpret_cast<const void*>(&dy::k_part_color), ctx->device, 128);
         d->coop_blocks_pgs = std::min(resident_blocks(dy::pgs_kernel(true), ctx->device), dy::kPgsBlocks);
-        // the reverse sweep keeps grid barriers between partitions
-        d->coop_blocks_adjoint = coop_blocks(reinterpret_cast<const void*>(&dy::k_pgs_adjoint), ctx->device);
+        d->coop_blocks_adjoint =
+            std::min(resident_blocks(reinterpret_cast<const void*>(&dy::k_pgs_adjoint), ctx->device), dy::kPgsBlocks);
         // room for the largest grid the autotuner may pick, and for the
         // tile sums of the degree scan
         d->blocksums.reserve(std::max<std::size_t>(2 * 1024 + 2, sel::tiles_for(static_cast<u32>(nb)) + 1));
