@@ -49,11 +49,12 @@ constexpr u32 kMaxParts = 4096;       // partitions per step
 constexpr u32 kMaxPending = 65536;    // managers left for overflow waves
 constexpr int kBlock = 256;
 constexpr int kCoopBlocks = 64;       // workgroups of the cooperative launches
+constexpr u32 kListRegs = 16;         // incidence lists up to this length are handled in registers
 constexpr int kPgsBlocks = 512;       // workgroups of the sweep (see k_pgs)
 
 // device counters
 enum : u32 { kFront0 = 0, kFront1, kFront2, kPend, kNParts, kPosIters, kVelIters, kRounds, kContacts, kFrictionRows,
-             kNbWord, kCtrWords = 16 };
+             kIncidence, kCtrWords = 16 };
 
 // The solver rows of the manager at a partition-sorted position, laid out
 // for the eight lanes that solve it (4 lanes per body: three components and
@@ -91,7 +92,7 @@ struct Ws {
     float4 *rpos, *rq;        // mass pose of the solver row
     float4* sii;              // 3 columns of the world sqrt inverse inertia
     u32* has_row;
-    u32 *deg, *off, *fill, *max_dyn, *body_mask;
+    u32 *deg, *off, *fill, *body_mask;  // incidence list of body b: inc[off[b]], deg[b] entries
     // per manager
     u32 *inc, *pred, *part, *pend, *sorted, *order;
     uint8_t* dd;  // [nm] the manager touches two dynamic bodies (a compact copy for the per-body passes)
@@ -219,19 +220,24 @@ __device__ inline bool manager_ok(const Ws& W, const fyzz_dy_manager& M) {
              M.count == 0 || M.count > 4);
 }
 
-// status flags and counters of the step (a fill kernel, so a captured
-// step records no memset node)
-__global__ __launch_bounds__(64) void k_clear(Ws W) {
-    if (threadIdx.x < kCtrWords) W.ctr[threadIdx.x] = 0;
-    if (threadIdx.x == 0) *W.flags = 0;
-    if (threadIdx.x < kBarWords && threadIdx.x != 1) W.bar[threadIdx.x] = 0;  // counts, not the generation
-}
-
-// scene.cpp:10383-10507 for default dynamics (no pending velocity mods)
+// Start of a step: status flags, counters, per-body and per-partition
+// counts cleared (plain stores, so a captured step records no memset
+// node), then the unconstrained velocities, scene.cpp:10383-10507 for
+// default dynamics (no pending velocity mods). The flags are raised from
+// the next kernel on (k_rows checks these velocities).
 __global__ __launch_bounds__(kBlock) void k_pre(Ws W) {
     const u32 i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < kCtrWords) W.ctr[i] = 0;
+    if (i == 0) *W.flags = 0;
+    if (i < kBarWords && i != 1) W.bar[i] = 0;  // counts, not the generation
+    if (i < kMaxParts) {
+        W.part_count[i] = 0;
+        W.part_fill[i] = 0;
+    }
     if (i >= W.nb) return;
     W.has_row[i] = 0;
+    W.deg[i] = 0;
+    W.fill[i] = 0;
     const fyzz_dy_body& b = W.bodies[i];
     if (b.flags & 1u) return;
     const float dt = W.dt;
@@ -266,32 +272,51 @@ __global__ __launch_bounds__(kBlock) void k_pre(Ws W) {
         a.y *= f;
         a.z *= f;
     }
-    if (!finite3(V{vx, vy, vz}) || !finite3(a)) raise_flag(W, FYZZ_DY_NONFINITE);
     W.pv[i] = make_float4(vx, vy, vz, 0.0f);
     W.pw[i] = make_float4(a.x, a.y, a.z, 0.0f);
 }
 
-// bodies of touching managers get a solver row (scene.cpp:6987-7013)
+// Bodies of touching managers get a solver row (scene.cpp:6987-7013);
+// incidence degrees (dynamic sides) and the manager's cleared entries for
+// the partitions.
 __global__ __launch_bounds__(kBlock) void k_mark(Ws W) {
     const u32 m = blockIdx.x * kBlock + threadIdx.x;
     if (m >= mcount(W)) return;
-    const fyzz_dy_manager M = W.mg[m];
-    if (!manager_ok(W, M)) {
+    const fyzz_dy_manager& M = W.mg[m];
+    W.part[m] = kNone;
+    W.entry[2 * m] = 0ull;
+    W.entry[2 * m + 1] = 0ull;
+    const bool ok = manager_ok(W, M);
+    W.dd[m] = ok && M.body0 >= 0 && M.body1 >= 0 ? 1u : 0u;
+    if (!ok) {
         raise_flag(W, FYZZ_DY_BAD_INPUT);
         return;
     }
-    if (M.body0 >= 0 && !(W.bodies[M.body0].flags & 1u)) W.has_row[M.body0] = 1;
-    if (M.body1 >= 0 && !(W.bodies[M.body1].flags & 1u)) W.has_row[M.body1] = 1;
+    if (M.body0 >= 0) {
+        atomicAdd(&W.deg[M.body0], 1u);
+        if (!(W.bodies[M.body0].flags & 1u)) W.has_row[M.body0] = 1;
+    }
+    if (M.body1 >= 0) {
+        atomicAdd(&W.deg[M.body1], 1u);
+        if (!(W.bodies[M.body1].flags & 1u)) W.has_row[M.body1] = 1;
+    }
 }
 
 // world sqrt inverse inertia R diag(sqrt I^-1) R^T (scene.cpp:7092-7110)
 __global__ __launch_bounds__(kBlock) void k_rows(Ws W) {
     // iteration counts (maximum over bodies with rows): one atomic per
     // workgroup and counter
-    __shared__ u32 pos_it, vel_it;
+    __shared__ u32 pos_it, vel_it, base;
+    __shared__ u32 scratch[kBlock / kWave + 1];
     if (threadIdx.x == 0) pos_it = vel_it = 0;
     __syncthreads();
     const u32 i = blockIdx.x * kBlock + threadIdx.x;
+    // the body's range of the incidence lists: the workgroup's bodies in
+    // order, the workgroups in any (a list is found by its offset and
+    // degree alone), so one counter takes the place of a scan's launches
+    u32 total;
+    const u32 before = block_exclusive_scan<kBlock>(i < W.nb ? W.deg[i] : 0u, scratch, &total);
+    if (threadIdx.x == 0) base = total ? atomicAdd(&W.ctr[kIncidence], total) : 0u;
     if (i < W.nb && W.has_row[i]) {
         const u32 it = W.bodies[i].iterations;
         atomicMax(&pos_it, it & 0xffu);
@@ -303,11 +328,22 @@ __global__ __launch_bounds__(kBlock) void k_rows(Ws W) {
         if (vel_it) atomicMax(&W.ctr[kVelIters], vel_it);
     }
     if (i >= W.nb) return;
+    W.off[i] = base + before;
+    const bool row = W.has_row[i];
+    {
+        // the sweep's state line: no change, no updates, the inverse mass
+        const u32 im = row ? __float_as_uint(W.bodies[i].inverse_mass) : 0u;
+        uint4* line = reinterpret_cast<uint4*>(W.vst + 8ull * i);
+        line[0] = line[1] = line[2] = make_uint4(0u, 0u, 0u, 0u);
+        line[3] = make_uint4(im, 0u, 0u, 0u);
+    }
+    if (!(W.bodies[i].flags & 1u) && (!finite3(f3(W.pv[i])) || !finite3(f3(W.pw[i]))))
+        raise_flag(W, FYZZ_DY_NONFINITE);
     float4 c0 = make_float4(0.f, 0.f, 0.f, 0.f), c1 = c0, c2 = c0;
     W.ang[i] = c0;
     W.mlin[i] = c0;
     W.mang[i] = c0;
-    if (!W.has_row[i]) {
+    if (!row) {
         W.lin[i] = c0;
         W.rpos[i] = c0;
         W.rq[i] = make_float4(0.f, 0.f, 0.f, 1.f);
@@ -369,44 +405,6 @@ __device__ inline bool dyn_dyn(const fyzz_dy_manager& M) { return M.body0 >= 0 &
 
 constexpr u64 kEntryReady = 1ull << 63;
 
-// per body: degree, CSR fill cursor, highest dynamic partition
-__global__ __launch_bounds__(kBlock) void k_part_clear(Ws W) {
-    const u32 i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < W.nb) {
-        W.deg[i] = 0;
-        W.fill[i] = 0;
-        W.max_dyn[i] = 0;
-#pragma unroll
-        for (u32 k = 0; k < 8; ++k) W.vst[8 * i + k] = 0ull;  // 0.0f, no updates yet
-        W.vst[8 * i + 6] = __float_as_uint(W.lin[i].w);       // the inverse mass (constant through the sweep)
-    }
-    if (i < kMaxParts) {
-        W.part_count[i] = 0;
-        W.part_fill[i] = 0;
-    }
-    if (i == 0) W.ctr[kNbWord] = W.nb;
-}
-
-// incidence degrees (dynamic sides); clears the manager's entries
-__global__ __launch_bounds__(kBlock) void k_part_degrees(Ws W) {
-    const u32 m = blockIdx.x * kBlock + threadIdx.x;
-    if (m >= mcount(W)) return;
-    const fyzz_dy_manager& M = W.mg[m];
-    W.part[m] = kNone;
-    W.entry[2 * m] = 0ull;
-    W.entry[2 * m + 1] = 0ull;
-    const bool ok = manager_ok(W, M);
-    W.dd[m] = ok && dyn_dyn(M) ? 1u : 0u;
-    if (!ok) return;
-    if (M.body0 >= 0) atomicAdd(&W.deg[M.body0], 1u);
-    if (M.body1 >= 0) atomicAdd(&W.deg[M.body1], 1u);
-}
-
-struct DegreeOf {
-    const u32* deg;
-    __device__ u32 operator()(u32 i) const { return deg[i]; }
-};
-
 // incidence lists, entry = manager << 1 | side
 __global__ __launch_bounds__(kBlock) void k_part_fill(Ws W) {
     const u32 m = blockIdx.x * kBlock + threadIdx.x;
@@ -417,27 +415,75 @@ __global__ __launch_bounds__(kBlock) void k_part_fill(Ws W) {
     if (M.body1 >= 0) W.inc[W.off[M.body1] + atomicAdd(&W.fill[M.body1], 1u)] = (m << 1) | 1u;
 }
 
+// One word of lane t (the same t in all lanes) in every lane.
+__device__ inline u32 lane_word(u32 x, u32 t) {
+    return static_cast<u32>(__builtin_amdgcn_readlane(static_cast<int>(x), static_cast<int>(t)));
+}
+
 // each body's list in manager order; predecessor links of the
 // dynamic/dynamic entries
+//
+// An insertion sort in place is a chain of dependent loads and stores, so
+// lists are ordered by counting, every load in flight at once: those of up
+// to kListRegs entries (almost all of a pile's) in one thread's registers,
+// those of up to a wave's width by the wave, a lane per entry. The longest
+// list of a launch set its time: a 30,000-box heap 21 -> 15 us.
 __global__ __launch_bounds__(kBlock) void k_part_chain(Ws W) {
     const u32 b = blockIdx.x * kBlock + threadIdx.x;
-    if (b >= W.nb) return;
-    const u32 lo = W.off[b], hi = W.off[b + 1];
-    for (u32 i = lo + 1; i < hi; ++i) {
-        const u32 e = W.inc[i];
-        u32 j = i;
-        while (j > lo && W.inc[j - 1] > e) {
-            W.inc[j] = W.inc[j - 1];
-            --j;
+    const u32 lo = b < W.nb ? W.off[b] : 0u, d = b < W.nb ? W.deg[b] : 0u, hi = lo + d;
+    for (u64 longs = __ballot(d > kListRegs && d <= kWave); longs; longs &= longs - 1) {
+        const u32 src = static_cast<u32>(__builtin_ctzll(longs));
+        const u32 at = lane_word(lo, src), len = lane_word(d, src), lane = lane_id();
+        const u32 e = lane < len ? W.inc[at + lane] : kNone;
+        const bool dyn = lane < len && W.dd[e >> 1];
+        const u64 dyns = __ballot(dyn);
+        u32 rank = 0, prev = 0;  // entry before + 1, 0: none
+        for (u32 t = 0; t < len; ++t) {
+            const u32 x = lane_word(e, t);
+            const bool less = x < e;
+            rank += less ? 1u : 0u;
+            prev = less && ((dyns >> t) & 1ull) ? max(prev, x + 1u) : prev;
         }
-        W.inc[j] = e;
+        if (lane < len) W.inc[at + rank] = e;
+        if (dyn) W.pred[e] = prev - 1u;
     }
-    u32 prev = kNone;
-    for (u32 i = lo; i < hi; ++i) {
-        const u32 e = W.inc[i];
-        if (!W.dd[e >> 1]) continue;
-        W.pred[e] = prev;
-        prev = e;
+    if (d <= kListRegs) {
+        u32 e[kListRegs], dyn = 0;
+#pragma unroll
+        for (u32 k = 0; k < kListRegs; ++k) e[k] = k < d ? W.inc[lo + k] : kNone;
+#pragma unroll
+        for (u32 k = 0; k < kListRegs; ++k)
+            if (k < d && W.dd[e[k] >> 1]) dyn |= 1u << k;
+#pragma unroll
+        for (u32 k = 0; k < kListRegs; ++k) {
+            if (k >= d) continue;
+            u32 rank = 0, prev = 0;  // as above
+#pragma unroll
+            for (u32 t = 0; t < kListRegs; ++t) {
+                const bool less = e[t] < e[k];  // (absent entries are never less)
+                rank += less ? 1u : 0u;
+                prev = less && ((dyn >> t) & 1u) ? max(prev, e[t] + 1u) : prev;
+            }
+            W.inc[lo + rank] = e[k];
+            if ((dyn >> k) & 1u) W.pred[e[k]] = prev - 1u;
+        }
+    } else if (d > kWave) {
+        for (u32 i = lo + 1; i < hi; ++i) {
+            const u32 e = W.inc[i];
+            u32 j = i;
+            while (j > lo && W.inc[j - 1] > e) {
+                W.inc[j] = W.inc[j - 1];
+                --j;
+            }
+            W.inc[j] = e;
+        }
+        u32 prev = kNone;
+        for (u32 i = lo; i < hi; ++i) {
+            const u32 e = W.inc[i];
+            if (!W.dd[e >> 1]) continue;
+            W.pred[e] = prev;
+            prev = e;
+        }
     }
 }
 
@@ -583,92 +629,103 @@ __global__ __launch_bounds__(kBlock) void k_part_color(Ws W) {
     }
 }
 
-// highest dynamic partition per body
-__global__ __launch_bounds__(kBlock) void k_part_maxdyn(Ws W) {
-    const u32 m = blockIdx.x * kBlock + threadIdx.x;
-    if (m >= mcount(W)) return;
-    const fyzz_dy_manager& M = W.mg[m];
-    if (!dyn_dyn(M)) return;
-    const u32 pm = W.part[m];
-    if (pm >= kPending) return;
-    atomicMax(&W.max_dyn[M.body0], pm + 1);
-    atomicMax(&W.max_dyn[M.body1], pm + 1);
-}
-
 // Dynamic/static managers follow the body's dynamic partitions; then each
 // of the body's managers is ranked by partition (the order in which a
 // sweep reaches them; a body's managers have distinct partitions). A
 // static manager touches one dynamic body, so this thread owns its
 // partition; the dynamic ones are final after the colouring.
+// Partition sizes are counted here too, each manager by its first dynamic
+// side: in LDS per workgroup first (a pile has a few tens of partitions, so
+// one global counter per manager would serialize ~10^4 atomics per
+// address), then one value per partition the workgroup holds.
 __global__ __launch_bounds__(kBlock) void k_part_static(Ws W) {
-    const u32 b = blockIdx.x * kBlock + threadIdx.x;
-    if (b >= W.nb) return;
-    const u32 lo = W.off[b], hi = W.off[b + 1];
-    u32 k = W.max_dyn[b];
-    // Bodies with at most kCache managers (all of a pile's) keep the
-    // partitions in registers: one load per manager instead of one per
-    // pair of managers. A static manager has this body as its only dynamic
-    // body, so this thread alone writes its partition.
-    constexpr u32 kCache = 16;
-    if (hi - lo <= kCache) {
-        u32 pc[kCache], ec[kCache];
-#pragma unroll
-        for (u32 q = 0; q < kCache; ++q) {
-            pc[q] = kNone;  // absent entries never count as lower
-            ec[q] = 0;
-            if (lo + q < hi) {
-                const u32 e = W.inc[lo + q];
-                const u32 m = e >> 1;
-                ec[q] = e;
-                if (!W.dd[m]) {
-                    W.part[m] = k;
-                    pc[q] = k++;
-                } else {
-                    pc[q] = W.part[m];
-                }
-            }
-        }
-#pragma unroll
-        for (u32 q = 0; q < kCache; ++q) {
-            if (lo + q >= hi) continue;
-            u32 r = 0;
-#pragma unroll
-            for (u32 t = 0; t < kCache; ++t) r += pc[t] < pc[q] ? 1u : 0u;
-            W.erank[ec[q]] = r;
-        }
-        return;
-    }
-    for (u32 i = lo; i < hi; ++i) {
-        const u32 m = W.inc[i] >> 1;
-        if (!W.dd[m]) W.part[m] = k++;
-    }
-    for (u32 i = lo; i < hi; ++i) {
-        const u32 e = W.inc[i];
-        const u32 pe = W.part[e >> 1];
-        u32 r = 0;
-        for (u32 j = lo; j < hi; ++j) r += W.part[W.inc[j] >> 1] < pe ? 1u : 0u;
-        W.erank[e] = r;
-    }
-}
-
-// Partition sizes and count. A pile has a few tens of partitions, so one
-// global counter per manager would serialize ~10^4 atomics per address:
-// each workgroup counts in LDS (its managers' partition range) and adds
-// one value per partition it holds.
-__global__ __launch_bounds__(kBlock) void k_part_sizes(Ws W) {
     __shared__ u32 cnt[kMaxParts];
     __shared__ u32 top;
-    const u32 m = blockIdx.x * kBlock + threadIdx.x;
     for (u32 i = threadIdx.x; i < kMaxParts; i += kBlock) cnt[i] = 0;
     if (threadIdx.x == 0) top = 0;
     __syncthreads();
-    const u32 pm = m < mcount(W) ? W.part[m] : kNone;
-    if (pm != kNone) {  // kNone: malformed record, already flagged
+    auto tally = [&](u32 pm) {
         if (pm >= kMaxParts) {
             raise_flag(W, FYZZ_DY_OVERFLOW);
         } else {
             atomicAdd(&cnt[pm], 1u);
             atomicMax(&top, pm + 1);
+        }
+    };
+    const u32 b = blockIdx.x * kBlock + threadIdx.x;
+    const u32 lo = b < W.nb ? W.off[b] : 0u, d = b < W.nb ? W.deg[b] : 0u, hi = lo + d;
+    // As in k_part_chain: a lane per manager for lists of up to a wave's
+    // width (a thread alone loads every pair of them: a 30,000-box heap
+    // 62 -> 17 us), registers for those of up to kListRegs.
+    for (u64 longs = __ballot(d > kListRegs && d <= kWave); longs; longs &= longs - 1) {
+        const u32 src = static_cast<u32>(__builtin_ctzll(longs));
+        const u32 at = lane_word(lo, src), len = lane_word(d, src), lane = lane_id();
+        const bool live = lane < len;
+        const u32 e = live ? W.inc[at + lane] : 0u, m = e >> 1;
+        const bool dyn = live && W.dd[m];
+        u32 pc = dyn ? W.part[m] : kNone;
+        u32 k = pc < kPending ? pc + 1u : 0u;
+        for (int o = kWave / 2; o > 0; o >>= 1) k = max(k, static_cast<u32>(__shfl_xor(static_cast<int>(k), o, kWave)));
+        const u64 stat = __ballot(live && !dyn);
+        if (live && !dyn) {
+            pc = k + lane_rank(stat);
+            W.part[m] = pc;
+        }
+        if (live && (!dyn || !(e & 1u))) tally(pc);
+        u32 r = 0;
+        for (u32 t = 0; t < len; ++t) r += lane_word(pc, t) < pc ? 1u : 0u;
+        if (live) W.erank[e] = r;
+    }
+    if (d <= kListRegs) {
+        u32 pc[kListRegs], ec[kListRegs], dyn = 0, k = 0;
+#pragma unroll
+        for (u32 q = 0; q < kListRegs; ++q) ec[q] = q < d ? W.inc[lo + q] : 0u;
+#pragma unroll
+        for (u32 q = 0; q < kListRegs; ++q) {
+            pc[q] = kNone;  // absent entries never count as lower
+            if (q < d && W.dd[ec[q] >> 1]) {
+                dyn |= 1u << q;
+                pc[q] = W.part[ec[q] >> 1];
+            }
+        }
+#pragma unroll
+        for (u32 q = 0; q < kListRegs; ++q)
+            if (pc[q] < kPending) k = max(k, pc[q] + 1u);
+#pragma unroll
+        for (u32 q = 0; q < kListRegs; ++q) {
+            if (q >= d) continue;
+            if (!((dyn >> q) & 1u)) {
+                W.part[ec[q] >> 1] = k;
+                pc[q] = k++;
+            }
+            if (!((dyn >> q) & 1u) || !(ec[q] & 1u)) tally(pc[q]);
+        }
+#pragma unroll
+        for (u32 q = 0; q < kListRegs; ++q) {
+            if (q >= d) continue;
+            u32 r = 0;
+#pragma unroll
+            for (u32 t = 0; t < kListRegs; ++t) r += pc[t] < pc[q] ? 1u : 0u;
+            W.erank[ec[q]] = r;
+        }
+    } else if (d > kWave) {
+        u32 k = 0;
+        for (u32 i = lo; i < hi; ++i) {
+            const u32 m = W.inc[i] >> 1;
+            if (W.dd[m] && W.part[m] < kPending) k = max(k, W.part[m] + 1u);
+        }
+        for (u32 i = lo; i < hi; ++i) {
+            const u32 e = W.inc[i], m = e >> 1;
+            const bool dyn = W.dd[m];
+            if (!dyn) W.part[m] = k++;
+            if (!dyn || !(e & 1u)) tally(W.part[m]);
+        }
+        for (u32 i = lo; i < hi; ++i) {
+            const u32 e = W.inc[i];
+            const u32 pe = W.part[e >> 1];
+            u32 r = 0;
+            for (u32 j = lo; j < hi; ++j) r += W.part[W.inc[j] >> 1] < pe ? 1u : 0u;
+            W.erank[e] = r;
         }
     }
     __syncthreads();
@@ -678,28 +735,29 @@ __global__ __launch_bounds__(kBlock) void k_part_sizes(Ws W) {
     if (threadIdx.x == 0 && np) atomicMax(&W.ctr[kNParts], np);
 }
 
-// partition offsets (one workgroup)
-__global__ __launch_bounds__(kBlock) void k_part_offsets(Ws W) {
-    __shared__ u32 scratch[kBlock / kWave + 1];
-    const u32 np = W.ctr[kNParts];
-    u32 carry = 0, total;
-    for (u32 t0 = 0; t0 < np; t0 += kBlock) {
-        const u32 t = t0 + threadIdx.x;
-        const u32 v = t < np ? W.part_count[t] : 0u;
-        const u32 ex = block_exclusive_scan<kBlock>(v, scratch, &total);
-        if (t < np) W.part_off[t] = carry + ex;
-        carry += total;
-    }
-    if (threadIdx.x == 0) W.part_off[np] = carry;
-}
-
 // Managers grouped by partition (order inside a partition is free): each
-// workgroup ranks its managers per partition in LDS, reserves one range
+// workgroup scans the partition sizes into offsets (the first one writes
+// them out), ranks its managers per partition in LDS, reserves one range
 // per partition it holds, then writes.
 __global__ __launch_bounds__(kBlock) void k_part_scatter(Ws W) {
     __shared__ u32 cnt[kMaxParts];
     __shared__ u32 base[kMaxParts];
     __shared__ u32 top;
+    __shared__ u32 scratch[kBlock / kWave + 1];
+    {
+        const u32 np = min(W.ctr[kNParts], kMaxParts);
+        u32 carry = 0, total;
+        for (u32 t0 = 0; t0 < np; t0 += kBlock) {
+            const u32 t = t0 + threadIdx.x;
+            const u32 ex = carry + block_exclusive_scan<kBlock>(t < np ? W.part_count[t] : 0u, scratch, &total);
+            if (t < np) {
+                base[t] = ex;
+                if (blockIdx.x == 0) W.part_off[t] = ex;
+            }
+            carry += total;
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) W.part_off[np] = carry;
+    }
     const u32 m = blockIdx.x * kBlock + threadIdx.x;
     for (u32 i = threadIdx.x; i < kMaxParts; i += kBlock) cnt[i] = 0;
     if (threadIdx.x == 0) top = 0;
@@ -714,7 +772,7 @@ __global__ __launch_bounds__(kBlock) void k_part_scatter(Ws W) {
     __syncthreads();
     const u32 np = top;
     for (u32 i = threadIdx.x; i < np; i += kBlock)
-        if (cnt[i]) base[i] = W.part_off[i] + atomicAdd(&W.part_fill[i], cnt[i]);
+        if (cnt[i]) base[i] += atomicAdd(&W.part_fill[i], cnt[i]);
     __syncthreads();
     if (live) {
         const fyzz_dy_manager& M = W.mg[m];
@@ -1866,7 +1924,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_bodies(Ws W) {
     V a_rows_v{0.f, 0.f, 0.f}, a_rows_w{0.f, 0.f, 0.f};
     float a_fric = 0.0f;
     if (mcount(W) && W.has_row[i]) {
-        for (u32 k = W.off[i]; k < W.off[i + 1]; ++k) {
+        for (u32 k = W.off[i]; k < W.off[i] + W.deg[i]; ++k) {
             const u32 e = W.inc[k], m = e >> 1, side = e & 1u;
             if (W.part[m] >= kMaxParts) continue;
             const float4 v = W.a_side[4 * m + 2 * side], w = W.a_side[4 * m + 2 * side + 1];
@@ -1975,9 +2033,7 @@ __device__ inline V apply_sii(V w, float4 c0, float4 c1, float4 c2, V s) {
 }
 
 // publish (scene.cpp:9509-9549), integrate and sleep check (10508-10707)
-__global__ __launch_bounds__(kBlock) void k_integrate(Ws W) {
-    const u32 i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= W.nb) return;
+__device__ void integrate_body(const Ws& W, u32 i) {
     fyzz_dy_body& B = W.bodies[i];
     if (B.flags & 1u) return;
     const float dt = W.dt;
@@ -2066,6 +2122,7 @@ __global__ __launch_bounds__(kBlock) void k_outputs(Ws W) {
     if (threadIdx.x == 0) s_rows = s_frows = 0;
     __syncthreads();
     const u32 m = blockIdx.x * kBlock + threadIdx.x;
+    if (W.with_rows && m < W.nb) integrate_body(W, m);
     u32 rows = 0, frows = 0;
     if (m < mcount(W)) {
         if (W.parts_out) W.parts_out[m] = W.part[m];
@@ -2073,7 +2130,8 @@ __global__ __launch_bounds__(kBlock) void k_outputs(Ws W) {
         if (W.with_rows && W.part[m] < kMaxParts) {
             const u32 o = W.order[m];
             const u32 no = min(o & 0xffu, 4u);
-            const float4 app = *reinterpret_cast<const float4*>(W.app + 8ull * W.pos_of[m]);
+            const u32 pos = W.pos_of[m];
+            const float4 app = *reinterpret_cast<const float4*>(W.app + 8ull * pos);
             const float applied[4] = {app.x, app.y, app.z, app.w};
 #pragma unroll
             for (u32 q = 0; q < 4; ++q) {
@@ -2084,7 +2142,7 @@ __global__ __launch_bounds__(kBlock) void k_outputs(Ws W) {
                 for (u32 k = 0; k < 4; ++k) out[k] = slot == k ? v : out[k];
             }
             rows = no;
-            frows = 2u * W.patches[m].anchor_count;
+            frows = 2u * ((static_cast<u32>(W.sinfo[pos].w) >> 8) & 0xffu);
         }
         if (W.impulses)
             for (u32 q = 0; q < 4; ++q) W.impulses[4 * m + q] = out[q];
@@ -2150,7 +2208,7 @@ struct fyzz_hip_dy {
     int coop_blocks_partition = 0, coop_blocks_pgs = 0, coop_blocks_adjoint = 0;
     bool plain_launch = false;
     DevBuf<float4> pv, pw, lin, ang, mlin, mang, rpos, rq, sii;
-    DevBuf<u32> has_row, deg, off, fill, max_dyn, body_mask;
+    DevBuf<u32> has_row, deg, off, fill, body_mask;
     DevBuf<u32> inc, pred, part, pend, sorted, order;
     DevBuf<uint8_t> dd;
     DevBuf<u64> entry;
@@ -2230,8 +2288,8 @@ void dy_prepare(fyzz_hip_dy* d, float dt, uint32_t nb, fyzz_dy_body* bodies, uin
     auto& prof = d->ctx->prof;
     {
         ProfScope ps(&prof, "dy.bodies", st);
-        hipLaunchKernelGGL(dy::k_clear, dim3(1), dim3(64), 0, st, w);
-        if (nb) hipLaunchKernelGGL(dy::k_pre, dim3(grid_for(nb, dy::kBlock)), dim3(dy::kBlock), 0, st, w);
+        hipLaunchKernelGGL(dy::k_pre, dim3(grid_for(std::max<u32>(nb, dy::kMaxParts), dy::kBlock)), dim3(dy::kBlock), 0,
+                           st, w);
         if (nm) hipLaunchKernelGGL(dy::k_mark, dim3(grid_for(nm, dy::kBlock)), dim3(dy::kBlock), 0, st, w);
         if (nb) hipLaunchKernelGGL(dy::k_rows, dim3(grid_for(nb, dy::kBlock)), dim3(dy::kBlock), 0, st, w);
         FYZZ_HIP_CHECK(hipGetLastError());
@@ -2239,24 +2297,16 @@ void dy_prepare(fyzz_hip_dy* d, float dt, uint32_t nb, fyzz_dy_body* bodies, uin
     {
         ProfScope ps(&prof, "dy.partition", st);
         const dim3 blk(dy::kBlock);
-        const dim3 gb(grid_for(std::max<u32>(nb, dy::kMaxParts), dy::kBlock)), gm(grid_for(nm, dy::kBlock));
-        hipLaunchKernelGGL(dy::k_part_clear, gb, blk, 0, st, w);
+        const dim3 gb(grid_for(std::max<u32>(nb, 1), dy::kBlock)), gm(grid_for(std::max<u32>(nm, 1), dy::kBlock));
         if (nm) {
-            hipLaunchKernelGGL(dy::k_part_degrees, gm, blk, 0, st, w);
-            if (nb)
-                sel::exclusive_scan(st, nb, d->ctr.get() + dy::kNbWord, dy::DegreeOf{d->deg.get()}, d->off.get(),
-                                    d->blocksums.get(), d->off.get() + nb);
             hipLaunchKernelGGL(dy::k_part_fill, gm, blk, 0, st, w);
-            if (nb) hipLaunchKernelGGL(dy::k_part_chain, dim3(grid_for(nb, dy::kBlock)), blk, 0, st, w);
+            hipLaunchKernelGGL(dy::k_part_chain, gb, blk, 0, st, w);
             FYZZ_HIP_CHECK(hipGetLastError());
             launch_coop(reinterpret_cast<const void*>(&dy::k_part_color), d->coop_blocks_partition, w, st,
                         d->plain_launch || !d->ctx->cooperative);
-            hipLaunchKernelGGL(dy::k_part_maxdyn, gm, blk, 0, st, w);
-            if (nb) hipLaunchKernelGGL(dy::k_part_static, dim3(grid_for(nb, dy::kBlock)), blk, 0, st, w);
-            hipLaunchKernelGGL(dy::k_part_sizes, gm, blk, 0, st, w);
+            hipLaunchKernelGGL(dy::k_part_static, gb, blk, 0, st, w);
         }
-        hipLaunchKernelGGL(dy::k_part_offsets, dim3(1), blk, 0, st, w);
-        if (nm) hipLaunchKernelGGL(dy::k_part_scatter, gm, blk, 0, st, w);
+        hipLaunchKernelGGL(dy::k_part_scatter, gm, blk, 0, st, w);
         FYZZ_HIP_CHECK(hipGetLastError());
     }
     if (!partition_only && nm) {
@@ -2282,10 +2332,8 @@ void dy_integrate(fyzz_hip_dy* d, float* impulses, uint32_t* partitions) {
     d->ws.impulses = impulses;
     d->ws.parts_out = partitions;
     ProfScope ps(&d->ctx->prof, "dy.integrate", st);
-    if (d->ws.nb)
-        hipLaunchKernelGGL(dy::k_integrate, dim3(grid_for(d->ws.nb, dy::kBlock)), dim3(dy::kBlock), 0, st, d->ws);
-    if (d->ws.nm)
-        hipLaunchKernelGGL(dy::k_outputs, dim3(grid_for(d->ws.nm, dy::kBlock)), dim3(dy::kBlock), 0, st, d->ws);
+    const u32 span = std::max(d->ws.nb, d->ws.nm);
+    if (span) hipLaunchKernelGGL(dy::k_outputs, dim3(grid_for(span, dy::kBlock)), dim3(dy::kBlock), 0, st, d->ws);
     FYZZ_HIP_CHECK(hipGetLastError());
     d->prepared = false;
 }
@@ -2395,8 +2443,7 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         const std::size_t nb = std::max<u32>(body_capacity, 1), nm = std::max<u32>(manager_capacity, 1);
         for (auto* b : {&d->pv, &d->pw, &d->lin, &d->ang, &d->mlin, &d->mang, &d->rpos, &d->rq}) b->reserve(nb);
         d->sii.reserve(3 * nb);
-        for (auto* b : {&d->has_row, &d->deg, &d->fill, &d->max_dyn, &d->body_mask}) b->reserve(nb);
-        d->off.reserve(nb + 1);
+        for (auto* b : {&d->has_row, &d->deg, &d->off, &d->fill, &d->body_mask}) b->reserve(nb);
         for (auto* b : {&d->inc, &d->pred}) b->reserve(2 * nm);
         d->entry.reserve(2 * nm);
         d->sinfo.reserve(nm);
@@ -2440,7 +2487,6 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         w.deg = d->deg.get();
         w.off = d->off.get();
         w.fill = d->fill.get();
-        w.max_dyn = d->max_dyn.get();
         w.body_mask = d->body_mask.get();
         w.inc = d->inc.get();
         w.pred = d->pred.get();
@@ -2467,7 +2513,7 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         w.bar = d->bar.get();
         // every workspace array the step kernels touch must exist
         const void* need[] = {w.pv, w.pw, w.lin, w.ang, w.mlin, w.mang, w.rpos, w.rq, w.sii, w.has_row,
-                              w.deg, w.off, w.fill, w.max_dyn, w.body_mask, w.inc, w.pred, w.part, w.pend,
+                              w.deg, w.off, w.fill, w.body_mask, w.inc, w.pred, w.part, w.pend,
                               w.sorted, w.order, w.entry, w.sinfo, w.srank, w.erank, w.vst, w.pos_of, w.rows,
                               w.app, w.fric,
                               w.part_count, w.part_off, w.part_fill, w.blocksums, w.ctr, w.flags, w.bar};
