@@ -38,6 +38,7 @@
 
 namespace fyzz_hip::sap {
 
+constexpr u32 kNone32 = 0xffffffffu;
 constexpr u64 kFoundBit = 1ull << 63;
 constexpr u64 kPairMask = ~kFoundBit;
 
@@ -65,9 +66,12 @@ enum Counter : u32 {
     kCounters
 };
 
-__global__ void k_fill(u32* p, u32 n, u32 v) {
+// Start of a frame: the per-frame counters cleared (the pair counts stay,
+// but `zero_pairs`'s on the first frame) and the moved bits.
+__global__ void k_reset(u32* cnt, u32 zero_pairs, u32* bits, u32 words) {
     const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+    if (i < kCounters && (i < kPairs0 || i >= kKept || i == zero_pairs)) cnt[i] = 0u;
+    if (i < words) bits[i] = 0u;
 }
 
 __global__ __launch_bounds__(256) void k_bounds_planes(u32 n, const float* pos, const float* quat,
@@ -1054,12 +1058,11 @@ void advance(Sap& s, const float* pos, const float* quat, const float* half, con
     const bool full = force_full || !s.built;
     const int nxt = s.cur ^ 1;
     u32* cnt = s.counters.p;
-    // reset the per-frame counters, keeping the current pair count
-    hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, cnt, static_cast<u32>(kPairs0), 0u);
-    hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, cnt + kKept, static_cast<u32>(kCounters - kKept), 0u);
     const u32 pairs_cur = s.cur == 0 ? kPairs0 : kPairs1;
     const u32 pairs_nxt = s.cur == 0 ? kPairs1 : kPairs0;
-    if (!s.built) hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, cnt + pairs_cur, 1u, 0u);
+    const u32 words = full ? 0u : (n + 31) / 32;
+    hipLaunchKernelGGL(k_reset, dim3(grid_for(std::max<u32>(words, kCounters), 256)), dim3(256), 0, st, cnt,
+                       s.built ? kNone32 : pairs_cur, s.moved_bits.p, words);
 
     Profiler* prof = &s.ctx->prof;
     {
@@ -1068,8 +1071,6 @@ void advance(Sap& s, const float* pos, const float* quat, const float* half, con
         if (n) hipLaunchKernelGGL(k_bounds_full, dim3(grid_for(n, 256)), dim3(256), 0, st, n, pos, quat, half, off,
                                   s.planes.p, s.rec_cur.p, s.coarse.p, stamp, cnt, s.sphere);
     } else {
-        const u32 words = (n + 31) / 32;
-        if (words) hipLaunchKernelGGL(k_fill, dim3(grid_for(words, 256)), dim3(256), 0, st, s.moved_bits.p, words, 0u);
         const u32 count = dirty ? n_dirty : n;
         if (count)
             hipLaunchKernelGGL(k_bounds_update, dim3(grid_for(count, 256)), dim3(256), 0, st, count, dirty, n, pos,

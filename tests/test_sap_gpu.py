@@ -57,6 +57,22 @@ def test_bounds_and_sort_match_oracle(ctx, orc, torch_cuda, n, seed):
     np.testing.assert_array_equal(u32(pays), wp)
 
 
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 1023, 1024, 1025, 2048, 2049, 4095, 4096, 4097, 8191, 8192, 8193])
+def test_endpoint_sort_at_the_one_launch_forms_edges(ctx, orc, torch_cuda, n):
+    """Sizes around the one-launch sort's items per thread (2, 4 and 8: up to
+    1,024, 2,048 and 4,096 boxes) and past its limit, keys with many ties in
+    every digit: exact order, ties by slot."""
+    from fyzz_amd import sap
+    torch = torch_cuda
+    rng = np.random.default_rng(n)
+    b = rng.integers(0, 2**32, (6, n), dtype=np.uint32) & np.uint32(0xC30F0180)
+    b[3:] |= np.uint32(1)  # as encoded, a min and a max key never tie
+    vals, pays = sap.sort_endpoints(ctx, dev(torch, b.view(np.int32)))
+    wv, wp = orc.sort_endpoints(b)
+    np.testing.assert_array_equal(u32(vals), wv)
+    np.testing.assert_array_equal(u32(pays), wp)
+
+
 def test_bounds_flags_nonfinite(ctx, torch_cuda):
     from fyzz_amd import sap
     torch = torch_cuda
