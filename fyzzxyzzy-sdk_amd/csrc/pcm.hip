@@ -1765,7 +1765,6 @@ void box_box_list(fyzz_hip_context* ctx, const ListPairs& L, const float* pos, c
     A.cache_src = static_cast<const Cache*>(L.cache_src);
     A.src_index = L.src_index;
     hipStream_t st = ctx->stream;
-    hipLaunchKernelGGL(k_zero1, dim3(1), dim3(1), 0, st, scratch);
     ProfScope ps(&ctx->prof, "pcm.box_box", st);
     hipLaunchKernelGGL(k_pcm_box_box, dim3(grid_for(L.cap, 128)), dim3(128), 0, st, A);
     hipLaunchKernelGGL(k_pcm_gjk, dim3(std::min<u32>(std::max<u32>(L.cap, 1u), 8192u)), dim3(64), 0, st, A);

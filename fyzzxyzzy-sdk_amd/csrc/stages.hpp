@@ -61,8 +61,9 @@ struct ListPairs {
     const u32* src_index;
     void* cache_dst;
 };
-// sphere: per slot, non-zero for a sphere of radius half[3 slot] (its
-// pairs take the stateless sphere contacts), or null when all are boxes.
+// scratch: the deferred pairs' count, which the caller has cleared on the
+// stream, then the list. sphere: per slot, non-zero for a sphere of radius
+// half[3 slot] (its pairs take the stateless sphere contacts), or null when all are boxes.
 void box_box_list(fyzz_hip_context* ctx, const ListPairs& L, const float* pos, const float* quat,
                   const float* half, float cd, float* contacts, u32* counts, u32* flags, u32* scratch,
                   const uint8_t* sphere = nullptr);

@@ -46,9 +46,19 @@ struct alignas(16) CacheRec {
     u32 w[kCacheWords];
 };
 
-__global__ void k_gather(u32 n, const fyzz_dy_body* bodies, float* pos, float* quat) {
+// Start of a step: the step number, the poses as the broadphase and the
+// narrowphase read them, the cleared per-box pair counts and links and the
+// deferred-pair count (one launch: each alone is a launch's latency).
+__global__ void k_begin(u32 n, const fyzz_dy_body* bodies, float* pos, float* quat, u32* counted, uint2* links,
+                        u32* d_step, u32* deferred) {
     const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        *d_step += 1u;
+        *deferred = 0u;
+    }
     if (i >= n) return;
+    counted[i] = 0u;
+    links[i] = make_uint2(kNone, kNone);
     const fyzz_dy_body& b = bodies[i];
     pos[3 * i] = b.position[0];
     pos[3 * i + 1] = b.position[1];
@@ -78,10 +88,12 @@ __device__ inline u32 lower_bound64(const u64* a, u32 n, u64 x) {
 // Gu order of a box/box pair (first = higher shape id, normals in the
 // second's frame), the pair's previous-list index (its cache and friction
 // history) and the broadphase pair count per box.
+// links: each dynamic box's first two pairs as the lower slot, for the
+// island pass (a static box joins no island).
 // known: the broadphase's own previous-list index of each pair (an
 // incremental frame records it), else found by a binary search.
 __global__ void k_pairs(u32 cap, const u64* cur, const u32* d_cur, const u64* prev, const u32* d_prev, u32* first,
-                        u32* second, u32* src, u32* counted, const u32* known, u32 n_dyn) {
+                        u32* second, u32* src, u32* counted, const u32* known, u32 n_dyn, uint2* links) {
     const u32 n = min(*d_cur, cap), np = min(*d_prev, cap);
     for (u32 t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
         const u64 x = cur[t];
@@ -98,19 +110,16 @@ __global__ void k_pairs(u32 cap, const u64* cur, const u32* d_cur, const u64* pr
             src[t] = (j < np && prev[j] == x) ? j : kNone;
         }
         atomicAdd(&counted[lo], 1u);
-        if (!stat) atomicAdd(&counted[hi], 1u);
+        if (!stat) {
+            atomicAdd(&counted[hi], 1u);
+            // the list is sorted by lower slot: a slot's first two pairs
+            const bool one = t == 0 || static_cast<u32>(cur[t - 1] >> 32) != lo;
+            if (one)
+                links[lo].x = hi;
+            else if (t == 1 || static_cast<u32>(cur[t - 2] >> 32) != lo)
+                links[lo].y = hi;
+        }
     }
-}
-
-__global__ void k_counted(u32 n, fyzz_dy_body* bodies, const u32* counted, u32 planes) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) bodies[i].counted_interactions = counted[i] + planes;
-}
-
-__global__ void k_step_begin(u32* d_step) { *d_step += 1u; }
-
-__global__ void k_total(const u32* d_nbb, u32 cap, u32 extra, u32* d_total) {
-    *d_total = min(*d_nbb, cap) + extra;
 }
 
 // A touching manager enters the solver list unless its island sleeps
@@ -229,18 +238,6 @@ __global__ void k_append_advance(const u32* d_nm, u32 cap_m, u64 capacity, u64* 
     const u64 c = *cursor;
     *count = n;
     *cursor = (c == ~0ull || c + n > capacity) ? ~0ull : c + n;
-}
-
-// friction patches solved this step, keyed for the next step's lookup
-__global__ void k_scatter_patches(const u32* d_nm, u32 cap_m, const fyzz_dy_patch* patches, const u32* mgr_slot,
-                                  fyzz_dy_patch* hist_next, u32* stamp_next, const u32* d_step) {
-    const u32 n = min(*d_nm, cap_m);
-    const u32 stamp = *d_step;
-    for (u32 m = blockIdx.x * blockDim.x + threadIdx.x; m < n; m += gridDim.x * blockDim.x) {
-        const u32 s = mgr_slot[m];
-        hist_next[s] = patches[m];
-        stamp_next[s] = stamp;
-    }
 }
 
 // ---- per-scene broadphase (independent scenes in one world)
@@ -589,31 +586,56 @@ __global__ void k_mgr_gather(const u32* order, u32 count, MgrWrite wr) {
     for (u32 o = blockIdx.x * blockDim.x + threadIdx.x; o < count; o += gridDim.x * blockDim.x) wr(order[o], o);
 }
 
-__global__ void k_touch(u32 cap, const u32* d_nbb, const u32* counts_bb, u32* touch_cur, u32 n, const u32* counts_pl,
-                        u32* touch_pl) {
-    const u32 nbb = min(*d_nbb, cap);
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < nbb || i < n; i += gridDim.x * blockDim.x) {
-        if (i < nbb) touch_cur[i] = counts_bb[i] != 0u ? 1u : 0u;
-        if (counts_pl && i < n) touch_pl[i] = counts_pl[i] != 0u ? 1u : 0u;
-    }
-}
 
+// End of a step: the friction patches solved in it, keyed for the next
+// step's lookup; the touching flags the next step compares with; and the
 // running totals over steps (algorithmic byte accounting of the solve):
 // [0] steps, [1] broadphase pairs, [2] managers, [3] contact rows,
 // [4] friction rows, [5] partitions, [6] position+velocity iterations,
 // [7] partition dependency depth, [8] broadphase found + lost pairs
-__global__ void k_accumulate(const u32* d_pairs, u32 cap, const u32* d_nm, const u32* dy_ctr, const u32* d_found,
-                             const u32* d_lost, u64* totals) {
-    totals[0] += 1;
-    totals[1] += min(*d_pairs, cap);
-    totals[2] += *d_nm;
-    totals[3] += dy_ctr[dy::kCtrContacts];
-    totals[4] += dy_ctr[dy::kCtrFriction];
-    totals[5] += dy_ctr[dy::kCtrParts];
-    totals[6] += dy_ctr[dy::kCtrPos] + max(dy_ctr[dy::kCtrVel], 1u);
-    totals[7] += dy_ctr[dy::kCtrRounds];
-    if (d_found) totals[8] += *d_found;
-    if (d_lost) totals[8] += *d_lost;
+struct EndArgs {
+    u32 cap, cap_m, n;
+    const u32* d_nbb;
+    const u32* d_nm;
+    const fyzz_dy_patch* patches;
+    const u32* mgr_slot;
+    fyzz_dy_patch* hist_next;
+    u32* stamp_next;
+    const u32* d_step;
+    const u32* counts_bb;
+    u32* touch_cur;
+    const u32* counts_pl;
+    u32* touch_pl;
+    const u32* dy_ctr;
+    const u32* d_found;
+    const u32* d_lost;
+    u64* totals;
+};
+__global__ void k_end(EndArgs A) {
+    const u32 nbb = min(*A.d_nbb, A.cap), nm = min(*A.d_nm, A.cap_m);
+    const u32 stamp = *A.d_step;
+    const u32 t0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    if (t0 == 0) {
+        A.totals[0] += 1;
+        A.totals[1] += nbb;
+        A.totals[2] += *A.d_nm;
+        A.totals[3] += A.dy_ctr[dy::kCtrContacts];
+        A.totals[4] += A.dy_ctr[dy::kCtrFriction];
+        A.totals[5] += A.dy_ctr[dy::kCtrParts];
+        A.totals[6] += A.dy_ctr[dy::kCtrPos] + max(A.dy_ctr[dy::kCtrVel], 1u);
+        A.totals[7] += A.dy_ctr[dy::kCtrRounds];
+        if (A.d_found) A.totals[8] += *A.d_found;
+        if (A.d_lost) A.totals[8] += *A.d_lost;
+    }
+    for (u32 m = t0; m < nm; m += stride) {
+        const u32 s = A.mgr_slot[m];
+        A.hist_next[s] = A.patches[m];
+        A.stamp_next[s] = stamp;
+    }
+    for (u32 i = t0; i < nbb || i < A.n; i += stride) {
+        if (i < nbb) A.touch_cur[i] = A.counts_bb[i] != 0u ? 1u : 0u;
+        if (A.counts_pl && i < A.n) A.touch_pl[i] = A.counts_pl[i] != 0u ? 1u : 0u;
+    }
 }
 
 // ---- islands: sleep and wake (Scene::activate_published_islands,
@@ -641,6 +663,7 @@ __global__ void k_accumulate(const u32* d_pairs, u32 cap, const u32* d_nm, const
 // counters, so the pass costs a few empty launches on steps where nothing
 // can sleep or wake, and it can be captured in a graph.
 constexpr u32 kSleeping = 1u, kReady = 2u, kActivating = 8u;
+constexpr u32 kLinkRounds = 5;  // rounds of k_isl_spec_link
 enum IslandCounter : u32 {
     kIslSleeping = 0,
     kIslActivating,
@@ -648,7 +671,8 @@ enum IslandCounter : u32 {
     kIslSleepingActivating,  // sleeping bodies carrying an activation (authored wakes)
     kIslMixed,               // speculative edges between a sleeping and an awake body
     kIslGiant,               // the largest speculative component after the link rounds (its root)
-    kIslCounters
+    kIslChanged,             // link round r hooked a root (kLinkRounds words)
+    kIslCounters = kIslChanged + 8
 };
 
 // Union-find on hardware whose L2 caches are not coherent across XCDs:
@@ -718,6 +742,12 @@ struct IslandArgs {
     u32* root_awake;       // per accurate root: a member is awake
     u32* ctr;              // kIslCounters
     uint8_t* asleep;       // per body: sleeping, as the pass found it (a compact copy for edge scans)
+    const u32* counted;    // per body: broadphase pairs
+    const uint2* links;    // per body: the upper slots of its first two pairs as the lower slot (kNone: none)
+    u32 planes;            // plane pairs per body
+    u32* d_total;          // out: candidates of the solver list (pairs + planes x bodies)
+    u32* bar;              // k_isl_pass: barrier arrivals, generation
+    u32* status;           // k_isl_pass: non-zero when its workgroups were not resident together
 };
 
 __device__ inline void set_bits(fyzz_dy_body& b, u32 on, u32 off) {
@@ -729,13 +759,16 @@ __device__ inline void set_bits(fyzz_dy_body& b, u32 on, u32 off) {
 // (activate_published_islands' first two loops): a pair found by the
 // broadphase activates both bodies unless both sleep; a touch found by
 // the narrowphase activates both and clears their readiness. Also resets
-// the union-find parents, the root flags and the counters for the pass.
+// the union-find parents, the root flags and the counters for the pass, and
+// writes each body's interaction count and the solver list's candidates.
 __global__ void k_isl_mark(IslandArgs A) {
     const u32 nbb = min(*A.d_cur, A.cap);
     const u32 stride = gridDim.x * blockDim.x;
     const u32 t0 = blockIdx.x * blockDim.x + threadIdx.x;
     if (t0 < kIslCounters) A.ctr[t0] = 0u;
+    if (t0 == 0) *A.d_total = nbb + (A.planes ? A.n : 0u);
     for (u32 i = t0; i < A.n; i += stride) {
+        A.bodies[i].counted_interactions = A.counted[i] + A.planes;
         A.spec[i] = i;
         A.acc[i] = i;
         A.root_wake[i] = 0u;
@@ -802,21 +835,13 @@ __device__ inline bool spec_needed(const IslandArgs& A) {
 __device__ inline u64 spec_edge(const IslandArgs& A, u32 i, u32 nbb) { return i < nbb ? A.cur[i] : A.gone[i - nbb]; }
 __device__ inline u32 edge_lo(u64 x) { return static_cast<u32>(x >> 32); }
 __device__ inline u32 edge_hi(u64 x) { return static_cast<u32>(x & 0xffffffffu); }
-// The link edges of the speculative union's first round: each body's
-// first two pairs as the lower slot (the list is sorted by lower slot).
-__device__ inline bool link_edge(const IslandArgs& A, u32 i, u32 nbb) {
-    if (i >= nbb) return false;
-    const u32 lo = edge_lo(A.cur[i]);
-    return i == 0 || edge_lo(A.cur[i - 1]) != lo || i == 1 || edge_lo(A.cur[i - 2]) != lo;
-}
-
 // Counts the edges between a sleeping and an awake body (sleep bits from
 // the compact per-body copy k_isl_count wrote).
-__global__ void k_isl_spec_mixed(IslandArgs A) {
+__device__ inline void isl_spec_mixed(const IslandArgs& A, u32 t0, u32 stride) {
     if (!wake_pass(A)) return;
     const u32 nbb = min(*A.d_cur, A.cap), ng = min(*A.d_gone, A.cap);
     u32 mixed = 0;
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < nbb + ng; i += gridDim.x * blockDim.x) {
+    for (u32 i = t0; i < nbb + ng; i += stride) {
         const u64 x = spec_edge(A, i, nbb);
         if (edge_hi(x) >= A.n) continue;  // a static body joins no island
         mixed += A.asleep[edge_lo(x)] != A.asleep[edge_hi(x)] ? 1u : 0u;
@@ -824,35 +849,85 @@ __global__ void k_isl_spec_mixed(IslandArgs A) {
     for (int d = kWave / 2; d > 0; d >>= 1) mixed += __shfl_xor(mixed, d, kWave);
     if (lane_id() == 0 && mixed) atomicAdd(&A.ctr[kIslMixed], mixed);
 }
+__global__ void k_isl_spec_mixed(IslandArgs A) { isl_spec_mixed(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x); }
 
-// When the components are needed: links each body to its first two pairs
-// (Afforest sampling: most bodies join one giant component through a
-// small share of the edges).
-__global__ void k_isl_spec_link(IslandArgs A) {
-    if (!spec_needed(A)) return;
-    const u32 nbb = min(*A.d_cur, A.cap);
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < nbb; i += gridDim.x * blockDim.x)
-        if (link_edge(A, i, nbb) && edge_hi(A.cur[i]) < A.n) unite(A.spec, edge_lo(A.cur[i]), edge_hi(A.cur[i]));
+// When the components are needed: one round of linking each body to its
+// first two pairs (Afforest sampling: most bodies join one giant component
+// through a small share of the edges). Two roots joined by an edge: the
+// larger is hooked under the smaller by an atomic minimum, so several hooks
+// of one root keep the smallest and a link lost to another is found in the
+// next one. Roots are read as they were when the round began: each round
+// is a launch (or follows a grid barrier), which makes the last one's hooks
+// visible. One asynchronous union instead walks L2 lines that the other
+// XCDs' hooks never refresh, one failed compare-and-swap per level: on the
+// formed pile of 100,000 boxes it took 280 us, the five rounds 95.
+// Of the bodies, one in this many links in a round (powers of two, another
+// subset each round). Once components are large, thousands of edges hook
+// the same few roots and their atomics serialize (a full third round took
+// 300 us on the pile, three later samples 66 together); a component needs
+// only one of its edges. The first round takes every body, so that the
+// samples meet components of several, and the last one joins what they
+// missed.
+__device__ inline u32 link_sample(u32 round) { return round == 1 ? 4u : round == 2 ? 32u : round == 3 ? 8u : 1u; }
+__device__ inline void isl_spec_link(const IslandArgs& A, u32 round, u32 t0, u32 stride) {
+    u32 hooked = 0;
+    const u32 every = link_sample(round);
+    // (every lane of a wave stays in the loop: the exchanges below read all)
+    for (u32 i0 = t0 - lane_id(); i0 < A.n; i0 += stride) {
+        const u32 i = i0 + lane_id();
+        const bool live = i < A.n;
+        uint2 l = live ? A.links[i] : make_uint2(kNone, kNone);
+        if (((i * 0x9E3779B1u) >> (8 + 4 * round)) & (every - 1u)) l = make_uint2(kNone, kNone);
+        const u32 p = live ? A.spec[i] : 0u;
+        const u32 x = live ? root_of(A.spec, p) : 0u;
+        if (live && x != p) A.spec[i] = x;  // (i is no root, so nothing hooks it)
+#pragma unroll
+        for (u32 side = 0; side < 2; ++side) {
+            const u32 o = side ? l.y : l.x;
+            const u32 y = o == kNone ? x : root_of(A.spec, o);
+            u32 hi = max(x, y), lo = min(x, y);
+            const bool differs = x != y;
+            // many edges hook one root once components are large: the
+            // wave's edges at its first lane's root become one
+            const u64 mask = __ballot(differs);
+            if (!mask) continue;
+            hooked = 1u;
+            const u32 first = static_cast<u32>(__builtin_ctzll(mask));
+            const u32 key = static_cast<u32>(__shfl(static_cast<int>(hi), static_cast<int>(first)));
+            const bool same = differs && hi == key;
+            u32 least = same ? lo : ~0u;
+            for (int d = kWave / 2; d > 0; d >>= 1)
+                least = min(least, static_cast<u32>(__shfl_xor(static_cast<int>(least), d, kWave)));
+            if (lane_id() == first) lo = least;
+            if (differs && (!same || lane_id() == first))
+                (void)__hip_atomic_fetch_min(&A.spec[hi], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if (__syncthreads_or(static_cast<int>(hooked)) && threadIdx.x == 0) A.ctr[kIslChanged + round] = 1u;
+}
+__global__ void k_isl_spec_link(IslandArgs A, u32 round) {
+    if (!spec_needed(A) || (round && !A.ctr[kIslChanged + round - 1])) return;
+    isl_spec_link(A, round, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 // Flattens the linked parents into labels.
-__global__ void k_isl_spec_compress(IslandArgs A) {
+__device__ inline void isl_spec_compress(const IslandArgs& A, u32 t0, u32 stride) {
     if (!spec_needed(A)) return;
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < A.n; i += gridDim.x * blockDim.x)
+    for (u32 i = t0; i < A.n; i += stride)
         A.spec[i] = root_of(A.spec, i);
 }
+__global__ void k_isl_spec_compress(IslandArgs A) { isl_spec_compress(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x); }
 
 // The most frequent label among 256 sampled bodies (one workgroup): the
 // giant component, whose internal edges the full union skips.
-__global__ void k_isl_spec_giant(IslandArgs A) {
-    if (!spec_needed(A)) return;
+__device__ inline u32 isl_spec_giant(const IslandArgs& A) {
     constexpr u32 kSamples = 256;
     __shared__ u32 lab[kSamples];
     for (u32 k = threadIdx.x; k < kSamples; k += blockDim.x)
         lab[k] = A.n ? A.spec[static_cast<u32>((static_cast<u64>(k) * A.n) / kSamples)] : 0u;
     __syncthreads();
     // count, for each sampled label, how often it occurs; keep the best
-    u32 best = 0u, best_count = 0u;
+    u32 best = ~0u, best_count = 0u;
     for (u32 k = threadIdx.x; k < kSamples; k += blockDim.x) {
         u32 c = 0;
         for (u32 j = 0; j < kSamples; ++j) c += lab[j] == lab[k] ? 1u : 0u;
@@ -867,17 +942,20 @@ __global__ void k_isl_spec_giant(IslandArgs A) {
     // largest count first, then smallest label
     atomicMin(&s_best, (static_cast<u64>(kSamples - best_count) << 32) | best);
     __syncthreads();
-    if (threadIdx.x == 0) A.ctr[kIslGiant] = static_cast<u32>(s_best & 0xffffffffu);
+    return static_cast<u32>(s_best & 0xffffffffu);
+}
+__global__ void k_isl_spec_giant(IslandArgs A) {
+    if (!spec_needed(A)) return;
+    const u32 g = isl_spec_giant(A);
+    if (threadIdx.x == 0) A.ctr[kIslGiant] = g;
 }
 
 // The full speculative union: every edge not already inside the giant
 // component (both labels equal the giant root: their bodies stay joined).
-__global__ void k_isl_union_spec(IslandArgs A) {
+__device__ inline void isl_union_spec(const IslandArgs& A, u32 giant, u32 t0, u32 stride) {
     if (!spec_needed(A)) return;
     const u32 nbb = min(*A.d_cur, A.cap), ng = min(*A.d_gone, A.cap);
-    const u32 giant = A.ctr[kIslGiant];
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < nbb + ng; i += gridDim.x * blockDim.x) {
-        if (link_edge(A, i, nbb)) continue;  // already united
+    for (u32 i = t0; i < nbb + ng; i += stride) {
         const u64 x = spec_edge(A, i, nbb);
         const u32 a = edge_lo(x), b = edge_hi(x);
         if (b >= A.n) continue;  // a static body joins no island
@@ -885,25 +963,27 @@ __global__ void k_isl_union_spec(IslandArgs A) {
         unite(A.spec, a, b);
     }
 }
+__global__ void k_isl_union_spec(IslandArgs A) { isl_union_spec(A, A.ctr[kIslGiant], blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x); }
 
 // Labels (flattened roots) and the roots of the speculative islands that
 // hold an activating body.
-__global__ void k_isl_wake_roots(IslandArgs A) {
+__device__ inline void isl_wake_roots(const IslandArgs& A, u32 t0, u32 stride) {
     if (!spec_needed(A)) return;
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < A.n; i += gridDim.x * blockDim.x) {
+    for (u32 i = t0; i < A.n; i += stride) {
         const u32 r = root_of(A.spec, i);
         if (A.bodies[i].flags & kActivating) A.root_wake[r] = 1u;
         A.spec[i] = r;
     }
 }
+__global__ void k_isl_wake_roots(IslandArgs A) { isl_wake_roots(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x); }
 
 // Wakes every sleeping member of those islands (wake counter 0.4 s at
 // least, readiness and sleep filter cleared) and consumes the activation
 // marks.
-__global__ void k_isl_wake(IslandArgs A) {
+__device__ inline void isl_wake(const IslandArgs& A, u32 t0, u32 stride) {
     if (A.ctr[kIslActivating] == 0u) return;
     const bool wake = spec_needed(A);
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < A.n; i += gridDim.x * blockDim.x) {
+    for (u32 i = t0; i < A.n; i += stride) {
         fyzz_dy_body& b = A.bodies[i];
         u32 f = b.flags & ~kActivating;
         if (wake && (f & kSleeping) && A.root_wake[root_of(A.spec, i)]) {
@@ -914,13 +994,14 @@ __global__ void k_isl_wake(IslandArgs A) {
         b.flags = f;
     }
 }
+__global__ void k_isl_wake(IslandArgs A) { isl_wake(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x); }
 
 // Accurate union over touches between two ready bodies; a touch between a
 // ready body and one that is not poisons the ready one.
-__global__ void k_isl_union_acc(IslandArgs A) {
+__device__ inline void isl_union_acc(const IslandArgs& A, u32 t0, u32 stride) {
     if (A.ctr[kIslReadyAwake] == 0u) return;
     const u32 nbb = min(*A.d_cur, A.cap);
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < nbb; i += gridDim.x * blockDim.x) {
+    for (u32 i = t0; i < nbb; i += stride) {
         if (A.counts_bb[i] == 0u) continue;
         const u32 a = A.first[i], b = A.second[i];
         if (b >= A.n) continue;  // touching a static body does not hold an island awake
@@ -931,11 +1012,12 @@ __global__ void k_isl_union_acc(IslandArgs A) {
             A.root_poison[ra ? a : b] = 1u;  // per body for now; folded into its root below
     }
 }
+__global__ void k_isl_union_acc(IslandArgs A) { isl_union_acc(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x); }
 
 // Per accurate component of ready bodies: poisoned, awake.
-__global__ void k_isl_sleep_roots(IslandArgs A) {
+__device__ inline void isl_sleep_roots(const IslandArgs& A, u32 t0, u32 stride) {
     if (A.ctr[kIslReadyAwake] == 0u) return;
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < A.n; i += gridDim.x * blockDim.x) {
+    for (u32 i = t0; i < A.n; i += stride) {
         const u32 f = A.bodies[i].flags;
         if (!(f & kReady)) continue;
         const u32 r = root_of(A.acc, i);
@@ -943,13 +1025,14 @@ __global__ void k_isl_sleep_roots(IslandArgs A) {
         if (!(f & kSleeping)) A.root_awake[r] = 1u;
     }
 }
+__global__ void k_isl_sleep_roots(IslandArgs A) { isl_sleep_roots(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x); }
 
 // A component of ready bodies that is a whole island (unpoisoned), with
 // one awake, goes to sleep: sleeping, wake counter 0, velocities and
 // sleep filter cleared.
-__global__ void k_isl_sleep(IslandArgs A) {
+__device__ inline void isl_sleep(const IslandArgs& A, u32 t0, u32 stride) {
     if (A.ctr[kIslReadyAwake] == 0u) return;
-    for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < A.n; i += gridDim.x * blockDim.x) {
+    for (u32 i = t0; i < A.n; i += stride) {
         fyzz_dy_body& b = A.bodies[i];
         const u32 f = b.flags;
         if ((f & (kReady | kSleeping)) != kReady) continue;
@@ -960,6 +1043,86 @@ __global__ void k_isl_sleep(IslandArgs A) {
         for (int k = 0; k < 3; ++k)
             b.linear_velocity[k] = b.angular_velocity[k] = b.sleep_linear_acc[k] = b.sleep_angular_acc[k] = 0.0f;
     }
+}
+__global__ void k_isl_sleep(IslandArgs A) { isl_sleep(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x); }
+
+// The pass from the mixed-edge count to the sleep in one launch of
+// kIslBlocks workgroups with a grid barrier between its phases (a plain
+// launch: every workgroup of so small a grid is resident; the barrier's
+// spin is bounded). The separate launches, most of them behind closed gates
+// on most steps, cost a launch's latency each (4.6 us in a replayed graph):
+// a 3,001-box heap takes 17 us here, 64 boxes 9. A barrier (5-10 us, with its L2 write-back and
+// invalidation) costs no less than a launch where the gates are open, and
+// 64 workgroups reach a quarter of the compute units, so larger worlds
+// keep the separate launches: the pile of 100,000 boxes 215 us in one
+// launch, 155 in separate ones.
+constexpr u32 kIslBlocks = 64;
+constexpr u32 kIslThreads = 1024;
+constexpr u32 kIslSpinLimit = 1u << 22;
+constexpr u32 kIslFusedMax = 16384;  // bodies up to which the one launch is taken
+
+__device__ inline void isl_grid_sync(const IslandArgs& A, u32& gen) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        const u32 g0 = gen;
+        if (__hip_atomic_fetch_add(&A.bar[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+            __hip_atomic_store(&A.bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
+            __hip_atomic_store(&A.bar[1], g0 + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            u32 spins = 0;
+            while (__hip_atomic_load(&A.bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g0) {
+                if (++spins > kIslSpinLimit) {
+                    atomicOr(A.status, 1u);
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        gen = g0 + 1u;
+    }
+    __syncthreads();
+}
+__device__ inline u32 isl_ctr(const IslandArgs& A, u32 k) {
+    return __hip_atomic_load(&A.ctr[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(kIslThreads) void k_isl_pass(IslandArgs A) {
+    const u32 activating = isl_ctr(A, kIslActivating), sleeping = isl_ctr(A, kIslSleeping);
+    const u32 ready_awake = isl_ctr(A, kIslReadyAwake);
+    if (!activating && !ready_awake) return;
+    const u32 t0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    u32 gen = threadIdx.x == 0 ? __hip_atomic_load(&A.bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    if (activating) {
+        if (sleeping) {
+            isl_spec_mixed(A, t0, stride);
+            isl_grid_sync(A, gen);
+        }
+        const bool spec = sleeping && (isl_ctr(A, kIslSleepingActivating) != 0u || isl_ctr(A, kIslMixed) != 0u);
+        if (spec) {
+            for (u32 r = 0; r < kLinkRounds; ++r) {
+                isl_spec_link(A, r, t0, stride);
+                isl_grid_sync(A, gen);
+                if (!isl_ctr(A, kIslChanged + r)) break;
+            }
+            for (u32 i = t0; i < A.n; i += stride) A.spec[i] = root_of(A.spec, i);
+            isl_grid_sync(A, gen);
+            isl_union_spec(A, isl_spec_giant(A), t0, stride);
+            isl_grid_sync(A, gen);
+            isl_wake_roots(A, t0, stride);
+            isl_grid_sync(A, gen);
+        }
+        isl_wake(A, t0, stride);
+    }
+    if (!ready_awake) return;
+    if (activating) isl_grid_sync(A, gen);
+    isl_union_acc(A, t0, stride);
+    isl_grid_sync(A, gen);
+    isl_sleep_roots(A, t0, stride);
+    isl_grid_sync(A, gen);
+    isl_sleep(A, t0, stride);
 }
 
 // ---- authored edits after the first step
@@ -1077,8 +1240,9 @@ struct fyzz_hip_world {
     DevBuf<fyzz_dy_patch> patches, hist[2];
     DevBuf<fyzz_friction_anchors> anchors;  // friction write-back, filled on demand
     // island pass: union-find parents (speculative, accurate), per-root flags, counters
-    DevBuf<u32> isl_spec, isl_acc, isl_root_wake, isl_root_poison, isl_root_awake, isl_ctr;
+    DevBuf<u32> isl_spec, isl_acc, isl_root_wake, isl_root_poison, isl_root_awake, isl_ctr, isl_bar;
     DevBuf<uint8_t> isl_asleep;
+    DevBuf<uint2> isl_links;
     DevBuf<u64> totals;
     DevBuf<u32> d_step;
     // graph stepping: one graph per parity of the double-buffer toggles
@@ -1243,6 +1407,9 @@ void upload(fyzz_hip_world* w) {
         b->reserve(nn);
     w->isl_ctr.reserve(world::kIslCounters);
     w->isl_asleep.reserve(nn);
+    w->isl_links.reserve(nn);
+    w->isl_bar.reserve(3);  // barrier words, then the status
+    FYZZ_HIP_CHECK(hipMemsetAsync(w->isl_bar.p, 0, 3 * sizeof(u32), st));
     w->totals.reserve(world::kTotals);
     FYZZ_HIP_CHECK(hipMemsetAsync(w->totals.p, 0, world::kTotals * sizeof(u64), st));
     w->d_step.reserve(1);
@@ -1488,20 +1655,26 @@ void islands(fyzz_hip_world* w, const sap::Lists& L, int c) {
                  gone,        d_gone,      w->src.p,       w->first.p,    w->second.p,
                  w->counts_bb.p, w->touch_bb[c].p, w->has_floor ? w->counts_pl.p : nullptr, w->touch_pl.p,
                  w->isl_spec.p, w->isl_acc.p, w->isl_root_wake.p, w->isl_root_poison.p, w->isl_root_awake.p,
-                 w->isl_ctr.p, w->isl_asleep.p};
+                 w->isl_ctr.p, w->isl_asleep.p, w->counted.p, w->isl_links.p, w->has_floor ? 1u : 0u, w->d_total.p, w->isl_bar.p,
+                 w->isl_bar.p + 2};
     const dim3 gp(std::min<u32>(grid_for(std::max(cap, n), 256), 2048u)), gb(std::min<u32>(grid_for(n, 256), 1024u));
     hipLaunchKernelGGL(k_isl_mark, gp, dim3(256), 0, st, A);
     hipLaunchKernelGGL(k_isl_count, gb, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_spec_mixed, gp, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_spec_link, gp, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_spec_compress, gb, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_spec_giant, dim3(1), dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_union_spec, gp, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_wake_roots, gb, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_wake, gb, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_union_acc, gp, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_sleep_roots, gb, dim3(256), 0, st, A);
-    hipLaunchKernelGGL(k_isl_sleep, gb, dim3(256), 0, st, A);
+    if (n <= kIslFusedMax) {
+        const u32 blocks = std::min<u32>(kIslBlocks, grid_for(cap, kIslThreads));
+        hipLaunchKernelGGL(k_isl_pass, dim3(blocks), dim3(kIslThreads), 0, st, A);
+    } else {
+        hipLaunchKernelGGL(k_isl_spec_mixed, gp, dim3(256), 0, st, A);
+        for (u32 r = 0; r < kLinkRounds; ++r) hipLaunchKernelGGL(k_isl_spec_link, gb, dim3(256), 0, st, A, r);
+        hipLaunchKernelGGL(k_isl_spec_compress, gb, dim3(256), 0, st, A);
+        hipLaunchKernelGGL(k_isl_spec_giant, dim3(1), dim3(256), 0, st, A);
+        hipLaunchKernelGGL(k_isl_union_spec, gp, dim3(256), 0, st, A);
+        hipLaunchKernelGGL(k_isl_wake_roots, gb, dim3(256), 0, st, A);
+        hipLaunchKernelGGL(k_isl_wake, gb, dim3(256), 0, st, A);
+        hipLaunchKernelGGL(k_isl_union_acc, gp, dim3(256), 0, st, A);
+        hipLaunchKernelGGL(k_isl_sleep_roots, gb, dim3(256), 0, st, A);
+        hipLaunchKernelGGL(k_isl_sleep, gb, dim3(256), 0, st, A);
+    }
     FYZZ_HIP_CHECK(hipGetLastError());
 }
 
@@ -1733,14 +1906,11 @@ void step(fyzz_hip_world* w, float dt) {
     ++w->step_index;
     if (!n) return;
     const u32 cap = w->pair_cap;
-    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, st, w->d_step.p);
-    hipLaunchKernelGGL(k_gather, dim3(grid_for(n, 256)), dim3(256), 0, st, n, w->bodies.p, w->pos.p, w->quat.p);
+    hipLaunchKernelGGL(k_begin, dim3(grid_for(n, 256)), dim3(256), 0, st, n, w->bodies.p, w->pos.p, w->quat.p,
+                       w->counted.p, w->isl_links.p, w->d_step.p, w->pcm_scratch.p);
     const sap::Lists L = w->n_scenes ? scene_broadphase(w) : sap_broadphase(w);
-    hipLaunchKernelGGL(k_fill, dim3(std::min<u32>(grid_for(n, 256), 1024u)), dim3(256), 0, st, w->counted.p, n, 0u);
     hipLaunchKernelGGL(k_pairs, dim3(std::min<u32>(grid_for(cap, 256), 4096u)), dim3(256), 0, st, cap, L.cur, L.d_cur,
-                       L.prev, L.d_prev, w->first.p, w->second.p, w->src.p, w->counted.p, L.src, n);
-    const u32 planes = w->has_floor ? 1u : 0u;
-    hipLaunchKernelGGL(k_counted, dim3(grid_for(n, 256)), dim3(256), 0, st, n, w->bodies.p, w->counted.p, planes);
+                       L.prev, L.d_prev, w->first.p, w->second.p, w->src.p, w->counted.p, L.src, n, w->isl_links.p);
     const int c = w->ccur, c2 = c ^ 1;  // previous / current pair-aligned buffers
     pcm::ListPairs lp{cap, L.d_cur, w->first.p, w->second.p, w->cache_bb[c].p, w->src.p, w->cache_bb[c2].p};
     const uint8_t* sphere = w->has_spheres ? w->sphere.p : nullptr;
@@ -1755,8 +1925,6 @@ void step(fyzz_hip_world* w, float dt) {
     islands(w, L, c);
     if (w->native_order) native_check_sleep(w);
     // touching managers, in order
-    const u32 extra = w->has_floor ? n : 0u;
-    hipLaunchKernelGGL(k_total, dim3(1), dim3(1), 0, st, L.d_cur, cap, extra, w->d_total.p);
     const int h = w->hcur;
     {
         ProfScope ps(&w->ctx->prof, "world.managers", st);
@@ -1775,15 +1943,11 @@ void step(fyzz_hip_world* w, float dt) {
     }
     dy::step_device(w->dy, dt, n, w->bodies.p, 1 + static_cast<u32>(w->host_statics.size()), w->statics.p, w->mgr_cap, w->d_nm.p, w->managers.p, w->hist[h].p,
                     w->mgr_cap, w->patches.p, w->impulses.p, w->parts.p);
-    hipLaunchKernelGGL(k_scatter_patches, dim3(std::min<u32>(grid_for(w->mgr_cap, 256), 2048u)), dim3(256), 0, st,
-                       w->d_nm.p, w->mgr_cap, w->patches.p, w->mgr_slot.p, w->hist[h ^ 1].p, w->stamp[h ^ 1].p,
-                       w->d_step.p);
-    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(1), 0, st, L.d_cur, cap, w->d_nm.p, dy::counters(w->dy),
-                       L.d_found, L.d_lost, w->totals.p);
     if (w->notify) publish_events(w, L, c, c2);
-    hipLaunchKernelGGL(k_touch, dim3(std::min<u32>(grid_for(std::max(cap, n), 256), 2048u)), dim3(256), 0, st, cap,
-                       L.d_cur, w->counts_bb.p, w->touch_bb[c2].p, n, w->has_floor ? w->counts_pl.p : nullptr,
-                       w->touch_pl.p);
+    EndArgs E{cap, w->mgr_cap, n, L.d_cur, w->d_nm.p, w->patches.p, w->mgr_slot.p, w->hist[h ^ 1].p,
+              w->stamp[h ^ 1].p, w->d_step.p, w->counts_bb.p, w->touch_bb[c2].p, w->has_floor ? w->counts_pl.p : nullptr,
+              w->touch_pl.p, dy::counters(w->dy), L.d_found, L.d_lost, w->totals.p};
+    hipLaunchKernelGGL(k_end, dim3(std::min<u32>(grid_for(std::max(w->mgr_cap, n), 256), 2048u)), dim3(256), 0, st, E);
     FYZZ_HIP_CHECK(hipGetLastError());
     w->hcur = h ^ 1;
 }
@@ -2384,7 +2548,7 @@ int fyzz_hip_world_stats(fyzz_hip_world* w, uint32_t* n_pairs, uint32_t* n_manag
     return guarded(w->ctx, [&] {
         u32 np = 0, nm = 0, parts = 0, dflags = 0, rounds = 0;
         if (w->uploaded && w->n) {
-            u32 err = 0, ovf = 0;
+            u32 err = 0, ovf = 0, isl = 0;
             sap::Lists L{};
             if (w->n_scenes) {
                 L.d_cur = w->scene_n.p + w->scur;
@@ -2398,8 +2562,9 @@ int fyzz_hip_world_stats(fyzz_hip_world* w, uint32_t* n_pairs, uint32_t* n_manag
             FYZZ_HIP_CHECK(hipMemcpyAsync(&err, L.d_error, 4, hipMemcpyDeviceToHost, st));
             FYZZ_HIP_CHECK(hipMemcpyAsync(&ovf, L.d_overflow, 4, hipMemcpyDeviceToHost, st));
             FYZZ_HIP_CHECK(hipMemcpyAsync(&nm, w->d_nm.p, 4, hipMemcpyDeviceToHost, st));
+            FYZZ_HIP_CHECK(hipMemcpyAsync(&isl, w->isl_bar.p + 2, 4, hipMemcpyDeviceToHost, st));
             (void)fyzz_hip_dy_status(w->dy, &dflags, &parts, &rounds);
-            dflags |= (err ? 0x100u : 0u) | (ovf ? 0x200u : 0u);
+            dflags |= (isl ? FYZZ_DY_LOGIC : 0u) | (err ? 0x100u : 0u) | (ovf ? 0x200u : 0u);
         }
         if (n_pairs) *n_pairs = np;
         if (n_managers) *n_managers = nm;

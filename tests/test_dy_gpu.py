@@ -135,6 +135,24 @@ def test_random_managers_two_steps_match_oracle(ctx, orc, torch_cuda, seed):
         mg, hist = with_history(mg, wp)
 
 
+@pytest.mark.parametrize("hub", [15, 16, 17, 63, 64, 65, 130])
+def test_incidence_lists_by_length_match_oracle(ctx, orc, torch_cuda, hub):
+    """Bodies whose contact lists sit at the edges of the forms that order
+    and rank them (up to 16 managers in one thread's registers, up to 64 by
+    a wave, longer in memory), several in one wave, with dynamic and static
+    managers in the same list: partitions exact, states as above."""
+    bodies, statics, mg = random_case(100 + hub, nb=300, n_dd=260, hub=hub, n_static=300, hubs=5)
+    odd = OracleDy(orc.lib)
+    solver = _solver(ctx, len(bodies), len(mg))
+    want, wp, wi, wparts = odd.step(1 / 120, bodies, statics, mg, np.zeros(0))
+    got, gp, gi, gparts, (flags, nparts, _) = _gpu_step(solver, 1 / 120, bodies, statics, mg, np.zeros(0))
+    assert flags == 0
+    np.testing.assert_array_equal(gparts, wparts)
+    np.testing.assert_allclose(body_state_from(got), body_state_from(want), rtol=RTOL, atol=ATOL)
+    np.testing.assert_allclose(gi, wi, rtol=RTOL, atol=1e-5)
+    np.testing.assert_array_equal(gp["anchor_count"], wp["anchor_count"])
+
+
 def test_free_fall_and_empty(ctx, orc, torch_cuda):
     """No managers: pre-integration and integration only (closed form)."""
     from fyzz_amd.dy import DY_MANAGER, DY_STATIC, default_bodies

@@ -57,3 +57,41 @@ def test_sleep_and_wake_match_reference(ctx, orc, torch_cuda, graph):
         assert w.stats()["flags"] == 0
     finally:
         w.close()
+
+
+@pytest.mark.parametrize("n_rows", [40, 1100])
+def test_island_pass_agrees_with_the_authority_on_long_rows(ctx, torch_cuda, n_rows):
+    """Rows of 15 resting boxes whose bounds touch (one broadphase island
+    each, one of them joined to a row of 600), slots in random order, go to
+    sleep; boxes dropped at staggered heights wake some rows. In the native
+    order every step compares the island pass's sleep flags with the host
+    authority's and fails on a difference. 40 rows take the one-launch pass
+    and 1,100 rows (17,100 boxes and more) the separate launches."""
+    from fyzz_amd.world import World
+    rng = np.random.default_rng(n_rows)
+    length = np.full(n_rows, 15)
+    length[0] = 600
+    row = np.repeat(np.arange(n_rows), length)
+    col = np.concatenate([np.arange(k) for k in length])
+    pos = np.stack([col * 1.01, np.full(len(row), 0.5), row * 3.0], 1)
+    drop = rng.choice(n_rows, n_rows // 4, replace=False)
+    fall = np.stack([rng.integers(0, 15, len(drop)) * 1.01, rng.uniform(6.0, 14.0, len(drop)), drop * 3.0], 1)
+    pos = np.concatenate([pos, fall]).astype(np.float32)
+    pos = pos[rng.permutation(len(pos))]
+    w = World(ctx, len(pos) + 1)
+    try:
+        fid = w.add_static_floor(0.0)
+        w.set_body_material(fid, 0.5, 0.5, 0.0)
+        w.add_dynamic_boxes(np.full((len(pos), 3), 0.5), pos, np.tile([0, 0, 0, 1.0], (len(pos), 1)), friction=0.5,
+                            restitution=0.0)
+        w.set_solver_order(True)
+        asleep = []
+        for s in range(230):
+            w.step(1 / 120)
+            if s % 10 == 9:
+                asleep.append(int((w.body_records()["flags"] & 1).sum()))
+        assert w.stats()["flags"] == 0
+        assert max(asleep) > len(pos) // 2
+        assert any(b < a for a, b in zip(asleep, asleep[1:]))  # rows woken by what fell on them
+    finally:
+        w.close()
