@@ -48,9 +48,11 @@ constexpr u32 kPending = 0xfffffffeu;
 constexpr u32 kMaxParts = 4096;       // partitions per step
 constexpr u32 kMaxPending = 65536;    // managers left for overflow waves
 constexpr int kBlock = 256;
-constexpr int kCoopBlocks = 64;       // workgroups of the cooperative launches
+constexpr int kColorBlocks = 256;     // workgroups of the colouring (64: +60 us on the pile, 1024: +27)
 constexpr u32 kListRegs = 16;         // incidence lists up to this length are handled in registers
 constexpr int kPgsBlocks = 512;       // workgroups of the sweep (see k_pgs)
+
+constexpr u32 kColorTicket = 0, kColorDone = 1, kBarWords = 2;
 
 // device counters
 enum : u32 { kFront0 = 0, kFront1, kFront2, kPend, kNParts, kPosIters, kVelIters, kRounds, kContacts, kFrictionRows,
@@ -107,10 +109,9 @@ struct Ws {
     float* app;     // [8 nm] applied impulses by position: 4 contact rows, 4 friction rows
     float4* fric;   // [nm] by position: the patch's static and dynamic friction, its flags
     u32 *part_count, *part_off, *part_fill;
-    u32* blocksums;
     u32* ctr;
     u32* flags;
-    u32* bar;  // grid barrier: arrival count, generation
+    u32* bar;  // the colouring's ticket and count of workgroups done
     // adjoint support (tape mode)
     u32 tape;             // record branches and raw row vectors
     u32 tape_iters;       // iterations the tape holds
@@ -135,57 +136,7 @@ struct Ws {
 __device__ inline u32 ld(const u32* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ inline void raise_flag(const Ws& W, u32 f) { atomicOr(W.flags, f); }
 __device__ inline u32 mcount(const Ws& W) { return W.d_nm ? min(ld(W.d_nm), W.nm) : W.nm; }
-// Grid-wide barrier of a cooperative launch (every workgroup resident),
-// two levels: workgroups arrive on their group's counter (groups of
-// kBarGroup), the last of each group arrives on the root counter, and the
-// last root arrival publishes the next generation. bar[0] root count,
-// bar[1] generation, bar[2 + g] group counts. Relaxed agent-scope atomics;
-// every workgroup releases its writes (agent scope) before arriving, the
-// releasing workgroup acquires before publishing, and every workgroup
-// acquires after leaving, so the grid's global-memory writes before the
-// barrier are visible after it. Thread 0 of each workgroup keeps the
-// generation it waits on. The spin is bounded; exceeding it (workgroups
-// not co-resident) raises a flag.
-constexpr u32 kSpinLimit = 1u << 20;
-constexpr u32 kBarGroup = 8;
-constexpr u32 kBarWords = 64;  // root, generation, up to 62 groups
-__device__ inline u32 barrier_start(const Ws& W) {
-    return threadIdx.x == 0 ? __hip_atomic_load(&W.bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-}
-__device__ inline void grid_sync(const Ws& W, u32& gen) {
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const u32 g0 = gen;
-        const u32 grp = blockIdx.x / kBarGroup;
-        const u32 ngroups = (gridDim.x + kBarGroup - 1) / kBarGroup;
-        const u32 gsize = min(kBarGroup, gridDim.x - grp * kBarGroup);
-        bool last = false;
-        if (__hip_atomic_fetch_add(&W.bar[2 + grp], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gsize - 1) {
-            __hip_atomic_store(&W.bar[2 + grp], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (__hip_atomic_fetch_add(&W.bar[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ngroups - 1) {
-                __hip_atomic_store(&W.bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                last = true;
-            }
-        }
-        if (last) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
-            __hip_atomic_store(&W.bar[1], g0 + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            u32 spins = 0;
-            while (__hip_atomic_load(&W.bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g0) {
-                if (++spins > kSpinLimit) {
-                    atomicOr(W.flags, FYZZ_DY_LOGIC);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        gen = g0 + 1u;
-    }
-    __syncthreads();
-}
+constexpr u32 kSpinLimit = 1u << 20;  // polls of one bounded wait; beyond it a status flag is raised
 // A wave whose lanes all wait backs off (64, 256, then 1024 cycles per
 // poll), so polling leaves the memory system to the waves doing work.
 __device__ inline void wait_backoff(u32 idle) {
@@ -229,7 +180,7 @@ __global__ __launch_bounds__(kBlock) void k_pre(Ws W) {
     const u32 i = blockIdx.x * kBlock + threadIdx.x;
     if (i < kCtrWords) W.ctr[i] = 0;
     if (i == 0) *W.flags = 0;
-    if (i < kBarWords && i != 1) W.bar[i] = 0;  // counts, not the generation
+    if (i < kBarWords) W.bar[i] = 0;
     if (i < kMaxParts) {
         W.part_count[i] = 0;
         W.part_fill[i] = 0;
@@ -522,71 +473,99 @@ __device__ void sort_pending(u32* a, u32 p) {
     }
 }
 
-// The colouring (cooperative) and the overflow waves.
+// The colouring and the overflow waves. A manager is coloured as soon as
+// the entries of its two predecessors are published. Workgroups take tiles
+// of kBlock managers by a ticket, so a tile's predecessors belong to it or
+// to tiles already taken by running workgroups: the colouring advances
+// however few of its workgroups are resident (a plain launch). The last
+// workgroup to finish runs the overflow waves.
+//
+// What bounds it: the chain of dependent managers. The list is sorted by
+// its lower slot, so most predecessors sit a few managers back: entries of
+// the tile are also kept in LDS, where a hop is a fraction of the trip
+// through memory, and a predecessor found ready is not polled again. With a
+// persistent thread per several managers, every hop through memory and a
+// grid barrier at the end (us): a 30,000-box heap 54, the formed pile of
+// 100,000 95, 1,024 stacks of 64 boxes 140; so 45, 58 and 76.
 __global__ __launch_bounds__(kBlock) void k_part_color(Ws W) {
-    u32 gen = barrier_start(W);
-    const u32 nthreads = gridDim.x * kBlock;
+    __shared__ u64 ent[2 * kBlock];
+    __shared__ u32 s_tile, s_depth, s_last;
     const u32 nm = mcount(W);
-    u32 m = blockIdx.x * kBlock + threadIdx.x;
-    bool have = false;
-    u32 p0 = kNone, p1 = kNone, spins = 0, depth = 0, idle = 0;
+    const u32 tiles = (nm + kBlock - 1) / kBlock;
+    if (threadIdx.x == 0) s_depth = 0;
+    bool pended = false;
     for (;;) {
-        bool progress = false;
-        if (m < nm && !have) {
-            if (!W.dd[m]) {  // not a valid manager between two dynamic bodies
-                m += nthreads;
-                progress = true;
-            } else {
-                p0 = W.pred[2 * m];
-                p1 = W.pred[2 * m + 1];
-                have = true;
-            }
-        }
-        if (m < nm && have) {
-            const u64 a0 = p0 != kNone ? __hip_atomic_load(&W.entry[p0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                       : kEntryReady;
-            const u64 a1 = p1 != kNone ? __hip_atomic_load(&W.entry[p1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                       : kEntryReady;
-            if ((a0 & kEntryReady) && (a1 & kEntryReady)) {
-                const u32 before0 = static_cast<u32>(a0), before1 = static_cast<u32>(a1);
-                const u32 level = max(static_cast<u32>(a0 >> 32) & 0x7fffffffu,
-                                      static_cast<u32>(a1 >> 32) & 0x7fffffffu) + 1u;
-                depth = max(depth, level);
-                const u32 avail = ~(before0 | before1);
-                u32 after0 = before0, after1 = before1;
-                if (avail) {
-                    const u32 bit = __builtin_ctz(avail);
-                    W.part[m] = bit;
-                    after0 |= 1u << bit;
-                    after1 |= 1u << bit;
-                } else {
-                    W.part[m] = kPending;
-                    const u32 k = atomicAdd(&W.ctr[kPend], 1u);
-                    if (k < kMaxPending) W.pend[k] = m;
+        if (threadIdx.x == 0) s_tile = atomicAdd(&W.bar[kColorTicket], 1u);
+        ent[threadIdx.x] = 0ull;
+        ent[kBlock + threadIdx.x] = 0ull;
+        __syncthreads();
+        const u32 tile = s_tile;
+        if (tile >= tiles) break;
+        const u32 first = tile * kBlock, m = first + threadIdx.x;
+        bool todo = m < nm && W.dd[m];  // a valid manager between two dynamic bodies
+        u32 p0 = todo ? W.pred[2 * m] : kNone, p1 = todo ? W.pred[2 * m + 1] : kNone;
+        u64 a0 = p0 == kNone ? kEntryReady : 0ull, a1 = p1 == kNone ? kEntryReady : 0ull;
+        const u32 base = 2 * first;
+        const bool local0 = p0 != kNone && p0 >= base, local1 = p1 != kNone && p1 >= base;
+        volatile u64* const vent = ent;
+        u32 spins = 0, idle = 0;
+        while (__ballot(todo)) {
+            bool progress = false;
+            if (todo) {
+                if (!a0)
+                    a0 = local0 ? vent[p0 - base]
+                                : __hip_atomic_load(&W.entry[p0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (!a1)
+                    a1 = local1 ? vent[p1 - base]
+                                : __hip_atomic_load(&W.entry[p1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (a0 && a1) {
+                    const u32 before0 = static_cast<u32>(a0), before1 = static_cast<u32>(a1);
+                    const u32 level = max(static_cast<u32>(a0 >> 32) & 0x7fffffffu,
+                                          static_cast<u32>(a1 >> 32) & 0x7fffffffu) + 1u;
+                    const u32 avail = ~(before0 | before1);
+                    const u32 bit = avail ? 1u << __builtin_ctz(avail) : 0u;
+                    const u64 hi = kEntryReady | (static_cast<u64>(level) << 32);
+                    const u64 e0 = hi | (before0 | bit), e1 = hi | (before1 | bit);
+                    vent[2 * threadIdx.x] = e0;
+                    vent[2 * threadIdx.x + 1] = e1;
+                    __hip_atomic_store(&W.entry[2 * m], e0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(&W.entry[2 * m + 1], e1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (avail) {
+                        W.part[m] = __builtin_ctz(avail);
+                    } else {
+                        W.part[m] = kPending;
+                        const u32 k = atomicAdd(&W.ctr[kPend], 1u);
+                        if (k < kMaxPending) W.pend[k] = m;
+                        pended = true;
+                    }
+                    atomicMax(&s_depth, level);
+                    todo = false;
+                    progress = true;
+                } else if (++spins > kSpinLimit) {
+                    // (the entries are published all the same, so that the
+                    // managers after this one do not wait for it in turn)
+                    raise_flag(W, FYZZ_DY_LOGIC);
+                    vent[2 * threadIdx.x] = vent[2 * threadIdx.x + 1] = kEntryReady;
+                    __hip_atomic_store(&W.entry[2 * m], kEntryReady, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(&W.entry[2 * m + 1], kEntryReady, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    todo = false;
                 }
-                const u64 hi = kEntryReady | (static_cast<u64>(level) << 32);
-                __hip_atomic_store(&W.entry[2 * m], hi | after0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&W.entry[2 * m + 1], hi | after1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                have = false;
-                m += nthreads;
-                progress = true;
-                spins = 0;  // the budget bounds one wait
-            } else if (++spins > kSpinLimit) {
-                raise_flag(W, FYZZ_DY_LOGIC);
-                m = nm;  // give up on this thread's managers
             }
+            idle = __ballot(progress) ? 0u : idle + 1u;
+            if (idle > 2u) wait_backoff(idle);
         }
-        const bool busy = m < nm;
-        if (!__ballot(busy)) break;
-        idle = __ballot(progress) ? 0u : idle + 1u;
-        wait_backoff(idle);
+        __syncthreads();
     }
-    // wave maximum first: one atomic per wave on the shared word
-    for (int d = kWave / 2; d > 0; d >>= 1) depth = max(depth, static_cast<u32>(__shfl_xor(static_cast<int>(depth), d, kWave)));
-    if (lane_id() == 0 && depth) atomicMax(&W.ctr[kRounds], depth);
-    grid_sync(W, gen);
+    // the pending list is written back before this workgroup counts as done
+    if (__syncthreads_or(pended)) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if (threadIdx.x == 0) {
+        if (s_depth > ld(&W.ctr[kRounds])) atomicMax(&W.ctr[kRounds], s_depth);
+        s_last = atomicAdd(&W.bar[kColorDone], 1u) == gridDim.x - 1 ? 1u : 0u;
+    }
+    __syncthreads();
+    if (!s_last || !ld(&W.ctr[kPend])) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     // overflow waves: the unassigned managers, in order, with fresh masks
-    if (blockIdx.x != 0) return;
     __shared__ u32 s_pending;
     if (threadIdx.x == 0) {
         u32 p = ld(&W.ctr[kPend]);
@@ -2218,7 +2197,7 @@ struct fyzz_hip_dy {
     DevBuf<u64> vst;
     DevBuf<float4> rows, fric;
     DevBuf<float> app;
-    DevBuf<u32> part_count, part_off, part_fill, blocksums, ctr, flags, bar;
+    DevBuf<u32> part_count, part_off, part_fill, ctr, flags, bar;
     // tape mode
     bool tape = false;
     bool taped_step = false;  // the last solved step recorded a tape
@@ -2238,13 +2217,6 @@ int resident_blocks(const void* kernel, int device) {
     FYZZ_REQUIRE(per_cu > 0 && cus > 0, kDeviceError, "dy: cooperative kernel does not fit a compute unit");
     return per_cu * cus;
 }
-int coop_blocks(const void* kernel, int device, int wanted = dy::kCoopBlocks) {
-    // 64 resident workgroups: a grid barrier costs ~3 us there, against
-    // ~17 us at 512 (the barrier is the Dy kernels' critical path)
-    // resident capacity, and the grid barrier's group counters
-    return std::min({resident_blocks(kernel, device), wanted, static_cast<int>(dy::kBarGroup * (dy::kBarWords - 2))});
-}
-
 // Cooperative launch (the runtime checks that every workgroup is resident).
 // Inside a captured graph the kernels are launched as plain kernels with
 // the same small grid (far below the device's resident capacity); the grid
@@ -2302,8 +2274,8 @@ void dy_prepare(fyzz_hip_dy* d, float dt, uint32_t nb, fyzz_dy_body* bodies, uin
             hipLaunchKernelGGL(dy::k_part_fill, gm, blk, 0, st, w);
             hipLaunchKernelGGL(dy::k_part_chain, gb, blk, 0, st, w);
             FYZZ_HIP_CHECK(hipGetLastError());
-            launch_coop(reinterpret_cast<const void*>(&dy::k_part_color), d->coop_blocks_partition, w, st,
-                        d->plain_launch || !d->ctx->cooperative);
+            hipLaunchKernelGGL(dy::k_part_color,
+                               dim3(std::min<u32>(d->coop_blocks_partition, grid_for(nm, dy::kBlock))), blk, 0, st, w);
             hipLaunchKernelGGL(dy::k_part_static, gb, blk, 0, st, w);
         }
         hipLaunchKernelGGL(dy::k_part_scatter, gm, blk, 0, st, w);
@@ -2397,20 +2369,17 @@ namespace fyzz_hip::dy {
 const u32* counters(fyzz_hip_dy* d) { return d->ctr.get(); }
 void set_plain_launch(fyzz_hip_dy* d, bool plain) { d->plain_launch = plain; }
 void set_coop_blocks(fyzz_hip_dy* d, int partition_blocks, int pgs_blocks) {
-    const int cap_p = coop_blocks(reinterpret_cast<const void*>(&k_part_color), d->ctx->device, 1 << 30);
+    const int cap_p = resident_blocks(reinterpret_cast<const void*>(&k_part_color), d->ctx->device);
     // the sweep has no grid barrier: its cap is the resident capacity
     const int cap_s = resident_blocks(pgs_kernel(true), d->ctx->device);
     FYZZ_REQUIRE(partition_blocks > 0 && pgs_blocks > 0, kInvalidArgument, "dy: workgroup counts must be positive");
     d->coop_blocks_partition = std::min(partition_blocks, cap_p);
     d->coop_blocks_pgs = std::min(pgs_blocks, cap_s);
-    FYZZ_REQUIRE(2 * static_cast<std::size_t>(std::max(d->coop_blocks_partition, d->coop_blocks_pgs)) + 2 <=
-                     d->blocksums.cap,
-                 kInvalidArgument, "dy: workgroup count beyond the workspace");
 }
 void effective_blocks(int device, int partition_blocks, int pgs_blocks, int* partition_out, int* pgs_out) {
-    const void* color = reinterpret_cast<const void*>(&k_part_color);
+    const int cap_p = resident_blocks(reinterpret_cast<const void*>(&k_part_color), device);
     const void* pgs = pgs_kernel(true);
-    *partition_out = partition_blocks > 0 ? coop_blocks(color, device, partition_blocks) : coop_blocks(color, device, 128);
+    *partition_out = std::min(partition_blocks > 0 ? partition_blocks : kColorBlocks, cap_p);
     *pgs_out = pgs_blocks > 0 ? std::min(pgs_blocks, resident_blocks(pgs, device)) : std::min(resident_blocks(pgs, device), kPgsBlocks);
 }
 void coop_blocks_of(fyzz_hip_dy* d, int* partition_blocks, int* pgs_blocks) {
@@ -2463,14 +2432,11 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         d->flags.reserve(1);
         d->bar.reserve(dy::kBarWords);
         FYZZ_HIP_CHECK(hipMemset(d->bar.get(), 0, dy::kBarWords * sizeof(u32)));
-        // 128 colouring workgroups measured best on the pile (64: +7 us, 256: +2 us)
-        d->coop_blocks_partition = coop_blocks(reinterpret_cast<const void*>(&dy::k_part_color), ctx->device, 128);
+        d->coop_blocks_partition =
+            std::min(resident_blocks(reinterpret_cast<const void*>(&dy::k_part_color), ctx->device), dy::kColorBlocks);
         d->coop_blocks_pgs = std::min(resident_blocks(dy::pgs_kernel(true), ctx->device), dy::kPgsBlocks);
         d->coop_blocks_adjoint =
             std::min(resident_blocks(reinterpret_cast<const void*>(&dy::k_pgs_adjoint), ctx->device), dy::kPgsBlocks);
-        // room for the largest grid the autotuner may pick, and for the
-        // tile sums of the degree scan
-        d->blocksums.reserve(std::max<std::size_t>(2 * 1024 + 2, sel::tiles_for(static_cast<u32>(nb)) + 1));
         FYZZ_HIP_CHECK(hipMemset(d->flags.get(), 0, sizeof(u32)));
         FYZZ_HIP_CHECK(hipMemset(d->ctr.get(), 0, dy::kCtrWords * sizeof(u32)));
         dy::Ws& w = d->ws;
@@ -2507,7 +2473,6 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
         w.part_count = d->part_count.get();
         w.part_off = d->part_off.get();
         w.part_fill = d->part_fill.get();
-        w.blocksums = d->blocksums.get();
         w.ctr = d->ctr.get();
         w.flags = d->flags.get();
         w.bar = d->bar.get();
@@ -2516,7 +2481,7 @@ int fyzz_hip_dy_create(fyzz_hip_context* ctx, uint32_t body_capacity, uint32_t m
                               w.deg, w.off, w.fill, w.body_mask, w.inc, w.pred, w.part, w.pend,
                               w.sorted, w.order, w.entry, w.sinfo, w.srank, w.erank, w.vst, w.pos_of, w.rows,
                               w.app, w.fric,
-                              w.part_count, w.part_off, w.part_fill, w.blocksums, w.ctr, w.flags, w.bar};
+                              w.part_count, w.part_off, w.part_fill, w.ctr, w.flags, w.bar};
         for (const void* q : need) FYZZ_REQUIRE(q != nullptr, kDeviceError, "dy_create: workspace array missing");
         *out = d.release();
     });

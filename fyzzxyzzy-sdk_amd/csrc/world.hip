@@ -2131,7 +2131,7 @@ int fyzz_hip_world_autotune(fyzz_hip_world* w, float dt, uint32_t trial_steps, i
         // increasing then decreasing order, and their two times are summed:
         // a drift linear in time adds the same to every candidate.
         constexpr int kCand = 5;
-        const int cand[kCand] = {16, 32, 64, 128, 256};
+        const int cand[kCand] = {64, 128, 256, 512, 1024};
         auto pick = [&](auto run) {
             float t[kCand] = {};
             for (int pass = 0; pass < 2; ++pass)
