@@ -62,7 +62,7 @@ enum Counter : u32 {
     kOverflow,  // a capacity was exceeded
     kSweep,
     kLarge,     // this frame's candidate list took the multi-workgroup sort
-    kLongWalks, // crossing walks handed to k_cross_long
+    kLongWalks, // gathered walks handed to k_cross_long_g
     kCounters
 };
 
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(256) void k_sweep(u32 n2, const u32* xpay, const Re
 // their relative order. For every endpoint e that moved from v to v', the
 // endpoints that crossed it have old or new positions inside [v, v'] (in
 // the total order): scan that interval in the new array and in the old
-// array. One wave per (moved box, axis); lanes stride over each interval.
+// array.
 // Every candidate pair is re-tested on all three axes with old and new
 // records; a status change emits the pair with kFoundBit for "found".
 // One crossing walk: the endpoint (a, kind) of a moved box on one axis,
@@ -355,131 +355,106 @@ struct CrossArgs {
     u64* out;
     u32* cnt;
     u32 cap;
-    u32* long_walks;   // walks still inside after kShortWalk entries
+    u32* long_walks;   // gathered walks still inside after kShortWalkG entries
     u32 long_cap;
     SplitArrays split;    // the gathered walks' kind-split arrays
 };
 
-// Entries a thread walks before handing the rest to a wave. Per-slot walks
-// start at random positions, so a thread's sequential steps are separate
-// line fetches, while a wave reads 64 consecutive entries per request
-// group: handing every walk that crosses more than one entry to a wave
-// measured fastest on 1M boxes at 10% moves (sap.pairs 1.40 ms at 16
-// entries, 1.03 at 4, 0.995 at 1).
-constexpr u32 kShortWalk = 1;
-
-// Walk geometry: the endpoint's rank, the bound (its other value) and the
-// direction. e sits at its new value in the new array and at its old value
-// in the old one; the crossed entries lie between e and the composite
-// (other value, pe), walking up or down from e.
+// Walk geometry: the bound (the endpoint's other value) and the direction.
+// e sits at its new value in the new array and at its old value in the old
+// one; the crossed entries lie between e and the composite (other value,
+// pe), walking up or down from e.
 struct WalkGeom {
-    const u32* K;
-    const u32* P;
-    u32 own, bound_v, pe;
+    u32 bound_v, pe;
     bool up;
 };
-__device__ inline WalkGeom walk_geom(const CrossArgs& A, const Walk& w, u32 v_old, u32 v_new) {
-    WalkGeom g;
-    const std::size_t ax = static_cast<std::size_t>(w.axis) * A.n2;
-    g.K = (w.arr ? A.old_key : A.new_key) + ax;
-    g.P = (w.arr ? A.old_pay : A.new_pay) + ax;
-    g.pe = (w.a << 1) | w.kind;
-    g.own = (w.arr ? A.old_rank : A.new_rank)[ax + g.pe];
-    g.bound_v = w.arr ? v_new : v_old;
-    g.up = (w.arr != 0) == (v_new > v_old);  // old array: toward v_new
-    return g;
-}
-// Is the step-th entry from e inside the crossed range? (j receives its
-// index and pj its payload, both loaded together)
-__device__ inline bool walk_inside(const CrossArgs& A, const WalkGeom& g, u32 step, u32& j, u32& pj) {
-    if (g.up) {
-        j = g.own + step;
-        if (j >= A.n2) return false;
-        const u32 kj = g.K[j];
-        pj = g.P[j];
-        return kj < g.bound_v || (kj == g.bound_v && pj < g.pe);
-    }
-    if (step > g.own) return false;
-    j = g.own - step;
-    const u32 kj = g.K[j];
-    pj = g.P[j];
-    return kj > g.bound_v || (kj == g.bound_v && pj > g.pe);
-}
-// A crossed entry (payload pf): a candidate pair when it is the other kind
-// of endpoint of another box; re-tested on all three axes with old and new
-// records. ca: the walking box's coarse bounds (its old and new keys). A
-// candidate whose coarse bounds miss them on some axis overlaps it neither
-// before nor after, so its status cannot change. The moved bit and the
-// coarse bounds are loaded together.
-__device__ inline void walk_visit(const CrossArgs& A, const Walk& w, u32 pf, const Rec& an, const Rec& ao,
-                                  const uint4& ca) {
-    const u32 b = pf >> 1;
-    if ((pf & 1u) == w.kind || b == w.a) return;
-    const u32 bits = A.moved_bits[b >> 5];
-    const uint4 cb = A.coarse[b];
-    const bool b_moved = (bits >> (b & 31u)) & 1u;
-    // an unmoved endpoint sits at the same value in both arrays: the
-    // new-array walk already saw it
-    if ((b_moved || !w.arr) && coarse_overlap(ca, cb)) {
-        const Rec bn = A.cur[b];
-        if (pair_allowed(an, bn)) {
-            const Rec bo = b_moved ? A.prev[b] : bn;
-            const bool ov_new = overlap3(an, bn);
-            const bool ov_old = overlap3(ao, bo);
-            if (ov_new != ov_old) emit(pair_key(w.a, b) | (ov_new ? kFoundBit : 0ull), A.out, A.cnt, kDelta, A.cap);
-        }
-    }
-}
 
-// One thread per walk (moved box x axis x endpoint kind x array) for its
-// first kShortWalk entries; longer walks continue in k_cross_long.
+// Per-slot walks (few boxes moved): one walk per moved box x axis x endpoint
+// kind x array. A wave takes 64 walks: each lane finds one walk's start and
+// bound, then groups of kWalkLanes lanes take the walks in turn, so that a
+// group's loads are consecutive entries and four walks are in flight.
+//
+// Every crossed entry of the other kind costs a look at its box. An unmoved
+// endpoint sits at the same value in both arrays, so the old-array walk
+// skips it, by the moved bit (a table that stays in L2) before the box's
+// coarse bounds (a random line): with a tenth of the boxes moved that is
+// nine of ten lines. The walks of 1,000,000 boxes, a tenth moved, a thread
+// for a walk's first entry and a wave for the rest: 948 us; this form 655
+// (8 lanes per walk 725, 32 635, at 1,000 boxes 10, 17 and 26 with 8, 16
+// and 32). What bounds it now: the random lines of the candidates' bounds.
+constexpr u32 kWalkLanes = 16;
 __global__ __launch_bounds__(256) void k_cross(CrossArgs A) {
+    const u32 lane = lane_id(), in_group = lane & (kWalkLanes - 1u), group = lane / kWalkLanes;
     const u32 n_work = min(*A.cnt_moved, A.n2 >> 1) * 12u;
-    for (u32 t = blockIdx.x * blockDim.x + threadIdx.x; t < n_work; t += gridDim.x * blockDim.x) {
-        const u32 wa = t >> 2;
-        const Walk w{A.moved[wa / 3u], wa % 3u, (t >> 1) & 1u, t & 1u};
-        const Rec an = A.cur[w.a];
-        const Rec ao = A.prev[w.a];
-        const u32 v_old = ao.k[w.axis + 3 * w.kind];
-        const u32 v_new = an.k[w.axis + 3 * w.kind];
-        if (v_old == v_new) continue;
-        const WalkGeom g = walk_geom(A, w, v_old, v_new);
-        const uint4 ca = A.coarse[w.a];
-        for (u32 step = 1;; ++step) {
-            u32 j, pj = 0;
-            if (!walk_inside(A, g, step, j, pj)) break;
-            walk_visit(A, w, pj, an, ao, ca);
-            if (step == kShortWalk) {
-                const u32 slot = atomicAdd(&A.cnt[kLongWalks], 1u);
-                if (slot < A.long_cap)
-                    A.long_walks[slot] = t;
-                else
-                    atomicOr(&A.cnt[kOverflow], 4u);
-                break;
+    const u32 n_waves = gridDim.x * (blockDim.x / kWave);
+    for (u32 base = (blockIdx.x * blockDim.x + threadIdx.x) / kWave * kWave; base < n_work; base += n_waves * kWave) {
+        // this lane's walk: where it starts, its bound, and packed
+        // (active, up, array, axis); its box's coarse bounds
+        u32 own = 0, bound_v = 0, pe = 0, how = 0;
+        uint4 ca = make_uint4(0u, 0u, 0u, 0u);
+        const u32 t = base + lane;
+        if (t < n_work) {
+            const u32 wa = t >> 2, axis = wa % 3u, kind = (t >> 1) & 1u, arr = t & 1u;
+            const u32 a = A.moved[wa / 3u];
+            const u32 v_old = A.prev[a].k[axis + 3 * kind], v_new = A.cur[a].k[axis + 3 * kind];
+            if (v_old != v_new) {
+                pe = (a << 1) | kind;
+                own = (arr ? A.old_rank : A.new_rank)[static_cast<std::size_t>(axis) * A.n2 + pe];
+                bound_v = arr ? v_new : v_old;
+                const u32 up = (arr != 0) == (v_new > v_old) ? 1u : 0u;  // old array: toward v_new
+                how = 1u | (up << 1) | (arr << 2) | (axis << 3);
+                ca = A.coarse[a];
             }
         }
-    }
-}
-
-// The rest of the long walks, one wave each, 64 entries per iteration
-// (sorted entries: the in-range lanes form a prefix).
-__global__ __launch_bounds__(256) void k_cross_long(CrossArgs A) {
-    const u32 lane = lane_id();
-    const u32 n_long = min(A.cnt[kLongWalks], A.long_cap);
-    const u32 n_waves = gridDim.x * (blockDim.x / kWave);
-    for (u32 i = (blockIdx.x * blockDim.x + threadIdx.x) / kWave; i < n_long; i += n_waves) {
-        const u32 t = A.long_walks[i];
-        const u32 wa = t >> 2;
-        const Walk w{A.moved[wa / 3u], wa % 3u, (t >> 1) & 1u, t & 1u};
-        const Rec an = A.cur[w.a];
-        const Rec ao = A.prev[w.a];
-        const WalkGeom g = walk_geom(A, w, ao.k[w.axis + 3 * w.kind], an.k[w.axis + 3 * w.kind]);
-        const uint4 ca = A.coarse[w.a];
-        for (u32 base = kShortWalk;; base += kWave) {
-            u32 j = 0, pj = 0;
-            const bool inside = walk_inside(A, g, base + lane + 1, j, pj);
-            if (inside) walk_visit(A, w, pj, an, ao, ca);
-            if (__ballot(inside) != ~0ull) break;
+        for (u32 g = 0; g < kWalkLanes; ++g) {
+            const int src = static_cast<int>(g * (kWave / kWalkLanes) + group);
+            const u32 w_how = static_cast<u32>(__shfl(static_cast<int>(how), src));
+            const u32 w_own = static_cast<u32>(__shfl(static_cast<int>(own), src));
+            const u32 w_pe = static_cast<u32>(__shfl(static_cast<int>(pe), src));
+            const u32 w_bound = static_cast<u32>(__shfl(static_cast<int>(bound_v), src));
+            const uint4 w_ca = make_uint4(static_cast<u32>(__shfl(static_cast<int>(ca.x), src)),
+                                          static_cast<u32>(__shfl(static_cast<int>(ca.y), src)),
+                                          static_cast<u32>(__shfl(static_cast<int>(ca.z), src)), 0u);
+            bool more = w_how & 1u;
+            const bool up = w_how & 2u, old = w_how & 4u;
+            const std::size_t ax = static_cast<std::size_t>(w_how >> 3) * A.n2;
+            const u32* const K = (old ? A.old_key : A.new_key) + ax;
+            const u32* const P = (old ? A.old_pay : A.new_pay) + ax;
+            const u32 a = w_pe >> 1;
+            for (u32 step = 1 + in_group; __ballot(more); step += kWalkLanes) {
+                // the step-th entry from e, while it is inside the crossed
+                // range (sorted: the lanes inside form a prefix)
+                bool inside = more && (up ? step < A.n2 - w_own : step <= w_own);
+                u32 pj = 0;
+                if (inside) {
+                    const u32 j = up ? w_own + step : w_own - step;
+                    const u32 kj = K[j];
+                    pj = P[j];
+                    inside = up ? kj < w_bound || (kj == w_bound && pj < w_pe)
+                                : kj > w_bound || (kj == w_bound && pj > w_pe);
+                }
+                more = more && inside;
+                // a crossed endpoint of the other kind, of another box: a
+                // candidate pair, re-tested on all three axes with old and
+                // new records when its coarse bounds (old and new keys)
+                // meet the walker's
+                const u32 b = pj >> 1;
+                if (inside && ((pj ^ w_pe) & 1u) && b != a) {
+                    const bool b_moved = (A.moved_bits[b >> 5] >> (b & 31u)) & 1u;
+                    if ((b_moved || !old) && coarse_overlap(w_ca, A.coarse[b])) {
+                        const Rec an = A.cur[a], bn = A.cur[b];
+                        if (pair_allowed(an, bn)) {
+                            const bool ov_new = overlap3(an, bn);
+                            const bool ov_old = overlap3(A.prev[a], b_moved ? A.prev[b] : bn);
+                            if (ov_new != ov_old)
+                                emit(pair_key(a, b) | (ov_new ? kFoundBit : 0ull), A.out, A.cnt, kDelta, A.cap);
+                        }
+                    }
+                }
+                // the group goes on while all of its lanes were inside
+                const u64 ins = __ballot(more) >> (group * kWalkLanes);
+                more = (ins & ((1ull << kWalkLanes) - 1ull)) == (1ull << kWalkLanes) - 1ull;
+            }
         }
     }
 }
@@ -561,16 +536,8 @@ __device__ inline bool walker_at(const CrossArgs& A, u32 t, Walk& w, u32& own) {
     w.kind = pe & 1u;
     return (A.moved_bits[w.a >> 5] >> (w.a & 31u)) & 1u;
 }
-__device__ inline WalkGeom walk_geom_at(const CrossArgs& A, const Walk& w, u32 own, u32 v_old, u32 v_new) {
-    WalkGeom g;
-    const std::size_t ax = static_cast<std::size_t>(w.axis) * A.n2;
-    g.K = (w.arr ? A.old_key : A.new_key) + ax;
-    g.P = (w.arr ? A.old_pay : A.new_pay) + ax;
-    g.pe = (w.a << 1) | w.kind;
-    g.own = own;
-    g.bound_v = w.arr ? v_new : v_old;
-    g.up = (w.arr != 0) == (v_new > v_old);
-    return g;
+__device__ inline WalkGeom walk_geom_at(const Walk& w, u32 v_old, u32 v_new) {
+    return {w.arr ? v_new : v_old, (w.a << 1) | w.kind, (w.arr != 0) == (v_new > v_old)};  // old array: toward v_new
 }
 __global__ __launch_bounds__(256) void k_cross_g(CrossArgs A) {
     const u32 n_work = 6u * A.n2;
@@ -583,7 +550,7 @@ __global__ __launch_bounds__(256) void k_cross_g(CrossArgs A) {
         const u32 v_old = ao.k[w.axis + 3 * w.kind];
         const u32 v_new = an.k[w.axis + 3 * w.kind];
         if (v_old == v_new) continue;
-        const WalkGeom g = walk_geom_at(A, w, own, v_old, v_new);
+        const WalkGeom g = walk_geom_at(w, v_old, v_new);
         const SplitWalk sw = split_walk(A, w, own);
         const uint2 ca = coarse_other(A.coarse[w.a], w.axis);
         for (u32 step = 1;; ++step) {
@@ -613,7 +580,7 @@ __global__ __launch_bounds__(256) void k_cross_long_g(CrossArgs A) {
         (void)walker_at(A, t, w, own);
         const Rec an = A.cur[w.a];
         const Rec ao = A.prev[w.a];
-        const WalkGeom g = walk_geom_at(A, w, own, ao.k[w.axis + 3 * w.kind], an.k[w.axis + 3 * w.kind]);
+        const WalkGeom g = walk_geom_at(w, ao.k[w.axis + 3 * w.kind], an.k[w.axis + 3 * w.kind]);
         const SplitWalk sw = split_walk(A, w, own);
         const uint2 ca = coarse_other(A.coarse[w.a], w.axis);
         for (u32 base = kShortWalkG;; base += kWave) {
@@ -1134,15 +1101,14 @@ void advance(Sap& s, const float* pos, const float* quat, const float* half, con
                     s.sorted_val[s.cur].p, s.rank[0].p, s.rank[1].p, s.moved_bits.p, s.rec_cur.p,
                     s.rec_prev.p, s.coarse.p, s.work_a.p, cnt, s.delta_cap, s.long_walks.p, 12u * n,
                     split};
-        const dim3 short_grid(std::min<u32>(grid_for(static_cast<std::size_t>(n) * 12, 256), 8192u));
+        const dim3 walk_grid(std::min<u32>(grid_for(std::max<std::size_t>(dirty ? n_dirty : n, 1) * 12, 256), 8192u));
         const dim3 sorted_grid(std::min<u32>(grid_for(6ull * n2, 256), 8192u));
         const dim3 long_grid(std::min<u32>(grid_for(static_cast<std::size_t>(n) * 12 * kWave, 256), 4096u));
         if (gather) {
             hipLaunchKernelGGL(k_cross_g, sorted_grid, dim3(256), 0, st, A);
             hipLaunchKernelGGL(k_cross_long_g, long_grid, dim3(256), 0, st, A);
         } else {
-            hipLaunchKernelGGL(k_cross, short_grid, dim3(256), 0, st, A);
-            hipLaunchKernelGGL(k_cross_long, long_grid, dim3(256), 0, st, A);
+            hipLaunchKernelGGL(k_cross, walk_grid, dim3(256), 0, st, A);
         }
         FYZZ_HIP_CHECK(hipGetLastError());
         prof->end("sap.pairs", pi, st);
