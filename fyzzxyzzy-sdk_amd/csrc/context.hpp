@@ -1,8 +1,11 @@
 // Library context: device, stream and the per-context error message that
 // the C-ABI reports through fyzz_hip_last_error().
 #pragma once
+#include <cstring>
 #include <exception>
+#include <initializer_list>
 #include <map>
+#include <mutex>
 #include <vector>
 #include <new>
 #include <string>
@@ -86,6 +89,36 @@ struct ProfScope {
         }
     }
 };
+// Pinned host memory for small readbacks: a copy into pageable memory is
+// staged by the runtime and synchronizes by itself, about 20 us each against
+// half of that into pinned memory. At most kMax bytes per context, given
+// back with it; larger readbacks go straight to the caller's memory.
+struct HostStage {
+    static constexpr std::size_t kMax = 1u << 20;
+    std::mutex mu;
+    unsigned char* p = nullptr;
+    std::size_t cap = 0;
+    ~HostStage() {
+        if (p) (void)hipHostFree(p);
+    }
+    void reserve(std::size_t n) {
+        if (n <= cap) return;
+        std::size_t want = 4096;
+        while (want < n) want <<= 1;
+        if (p) FYZZ_HIP_CHECK(hipHostFree(p));
+        p = nullptr;
+        cap = 0;
+        void* q = nullptr;
+        FYZZ_HIP_CHECK(hipHostMalloc(&q, want, hipHostMallocDefault));
+        p = static_cast<unsigned char*>(q);
+        cap = want;
+    }
+};
+struct Readback {
+    void* dst;        // host
+    const void* src;  // device
+    std::size_t bytes;
+};
 }  // namespace fyzz_hip
 
 struct fyzz_hip_context {
@@ -94,9 +127,41 @@ struct fyzz_hip_context {
     bool cooperative = true;       // grid-barrier kernels: cooperative or plain launches
     std::string last_error;
     fyzz_hip::Profiler prof;
+    fyzz_hip::HostStage stage;
 };
 
 namespace fyzz_hip {
+
+// Device words read back in stream order with one synchronization.
+inline void read_back(fyzz_hip_context* ctx, std::initializer_list<Readback> parts) {
+    hipStream_t st = ctx->stream;
+    std::size_t total = 0;
+    for (const Readback& r : parts) total += (r.bytes + 15) & ~std::size_t{15};
+    if (total > HostStage::kMax) {
+        for (const Readback& r : parts)
+            if (r.bytes) FYZZ_HIP_CHECK(hipMemcpyAsync(r.dst, r.src, r.bytes, hipMemcpyDeviceToHost, st));
+        FYZZ_HIP_CHECK(hipStreamSynchronize(st));
+        return;
+    }
+    if (!total) {
+        FYZZ_HIP_CHECK(hipStreamSynchronize(st));
+        return;
+    }
+    std::lock_guard<std::mutex> lock(ctx->stage.mu);
+    ctx->stage.reserve(total);
+    std::size_t at = 0;
+    for (const Readback& r : parts) {
+        if (r.bytes)
+            FYZZ_HIP_CHECK(hipMemcpyAsync(ctx->stage.p + at, r.src, r.bytes, hipMemcpyDeviceToHost, st));
+        at += (r.bytes + 15) & ~std::size_t{15};
+    }
+    FYZZ_HIP_CHECK(hipStreamSynchronize(st));
+    at = 0;
+    for (const Readback& r : parts) {
+        if (r.bytes) std::memcpy(r.dst, ctx->stage.p + at, r.bytes);
+        at += (r.bytes + 15) & ~std::size_t{15};
+    }
+}
 
 // Runs f, converting exceptions into a status code and the context's
 // last-error string; no exception crosses the C-ABI.

@@ -918,18 +918,33 @@ __global__ __launch_bounds__(kListThreads) void k_lists(const u64* d_in, u64* tm
     }
 }
 
+enum HostWord : u32 { kHostPairs, kHostFound, kHostLost, kHostError, kHostOverflow, kHostFrame, kHostWords };
+
 // new list = (old - lost) + found in one pass: lost is a subset of old and
 // found is disjoint from it, so every output position is a rank sum.
 // src[pos]: the new pair's index in the old list (kNone: found this frame),
 // which the caller would otherwise find by a binary search per pair.
 __global__ void k_apply_delta(u32 cap, const u64* old, const u32* d_no, const u64* found, const u32* d_nf,
-                              const u64* lost, const u32* d_nl, u64* out, u32* d_nout, u32* cnt, u32* src) {
+                              const u64* lost, const u32* d_nl, u64* out, u32* d_nout, u32* cnt, u32* src,
+                              u32* host, u32 frame) {
     const u32 no = *d_no, nf = *d_nf, nl = *d_nl;
     const u32 total = no - nl + nf;
     const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {
         *d_nout = min(total, cap);
-        if (total > cap) atomicOr(&cnt[kOverflow], 2u);
+        const u32 over = cnt[kOverflow] | (total > cap ? 2u : 0u);
+        if (total > cap) cnt[kOverflow] = over;
+        if (host) {
+            // the frame's counts in pinned host memory (this launch is the
+            // last to touch them), so that reading them takes a
+            // synchronization and no copy
+            host[kHostPairs] = min(total, cap);
+            host[kHostFound] = nf;
+            host[kHostLost] = nl;
+            host[kHostError] = cnt[kError];
+            host[kHostOverflow] = over;
+            host[kHostFrame] = frame;
+        }
     }
     for (u32 i = t; i < no + nf; i += gridDim.x * blockDim.x) {
         u32 pos, from;
@@ -974,7 +989,13 @@ struct Sap {
     bool src_valid = false;  // the last frame was incremental, so src is current
     const uint8_t* sphere = nullptr;  // per slot: a sphere (set by the world), or null
     std::vector<u32> host_counters;
+    // pinned words the incremental frames publish their counts to (from the
+    // first time the counts are asked for)
+    u32* host_words = nullptr;
 
+    ~Sap() {
+        if (host_words) (void)hipHostFree(host_words);
+    }
     u32 list_cap() const { return std::max(pair_cap, delta_cap); }
 };
 
@@ -1119,7 +1140,7 @@ void advance(Sap& s, const float* pos, const float* quat, const float* half, con
                            cnt + kDelta, s.delta_cap, s.found.p, s.lost.p, cnt, s.list_bar.p, slot_bits - 6);
         hipLaunchKernelGGL(k_apply_delta, dim3(std::min<u32>(grid_for(static_cast<std::size_t>(s.pair_cap) + s.delta_cap, 256), 2048u)), dim3(256), 0, st,
                            s.pair_cap, s.pairs[s.cur].p, cnt + pairs_cur, s.found.p, cnt + kFound, s.lost.p,
-                           cnt + kLost, s.pairs[nxt].p, cnt + pairs_nxt, cnt, s.src.p);
+                           cnt + kLost, s.pairs[nxt].p, cnt + pairs_nxt, cnt, s.src.p, s.host_words, stamp);
     }
     FYZZ_HIP_CHECK(hipGetLastError());
     s.cur = nxt;
@@ -1314,10 +1335,24 @@ int fyzz_hip_sap_counts(fyzz_hip_sap* sap, uint64_t* n_pairs, uint64_t* n_found,
     if (!sap) return kInvalidArgument;
     return guarded(sap->s.ctx, [&] {
         sap::Sap& s = sap->s;
+        if (s.host_words) {
+            FYZZ_HIP_CHECK(hipStreamSynchronize(s.ctx->stream));
+            const volatile u32* h = s.host_words;
+            if (s.src_valid && h[sap::kHostFrame] == s.frame) {
+                if (n_pairs) *n_pairs = h[sap::kHostPairs];
+                if (n_found) *n_found = h[sap::kHostFound];
+                if (n_lost) *n_lost = h[sap::kHostLost];
+                if (status_flags) *status_flags = (h[sap::kHostError] ? 1u : 0u) | (h[sap::kHostOverflow] ? 2u : 0u);
+                return;
+            }
+        } else {
+            void* p = nullptr;
+            FYZZ_HIP_CHECK(hipHostMalloc(&p, sap::kHostWords * sizeof(u32), hipHostMallocDefault));
+            s.host_words = static_cast<u32*>(p);
+            std::fill(s.host_words, s.host_words + sap::kHostWords, 0u);
+        }
         s.host_counters.resize(sap::kCounters);
-        FYZZ_HIP_CHECK(hipMemcpyAsync(s.host_counters.data(), s.counters.p, sizeof(u32) * sap::kCounters,
-                                      hipMemcpyDeviceToHost, s.ctx->stream));
-        FYZZ_HIP_CHECK(hipStreamSynchronize(s.ctx->stream));
+        read_back(s.ctx, {{s.host_counters.data(), s.counters.p, sizeof(u32) * sap::kCounters}});
         const auto& c = s.host_counters;
         if (n_pairs) *n_pairs = c[s.cur == 0 ? sap::kPairs0 : sap::kPairs1];
         if (n_found) *n_found = c[sap::kFound];
@@ -1343,8 +1378,7 @@ int fyzz_hip_sap_fetch(fyzz_hip_sap* sap, int which, uint32_t* out_pairs, uint64
         const uint64_t n = which == 0 ? np : which == 1 ? nf : nl;
         const uint64_t m = std::min<uint64_t>(n, capacity);
         std::vector<u64> tmp(m);
-        if (m) FYZZ_HIP_CHECK(hipMemcpyAsync(tmp.data(), src, sizeof(u64) * m, hipMemcpyDeviceToHost, s.ctx->stream));
-        FYZZ_HIP_CHECK(hipStreamSynchronize(s.ctx->stream));
+        if (m) read_back(s.ctx, {{tmp.data(), src, sizeof(u64) * m}});
         for (uint64_t i = 0; i < m; ++i) {
             out_pairs[2 * i] = static_cast<u32>(tmp[i] >> 32);
             out_pairs[2 * i + 1] = static_cast<u32>(tmp[i] & 0xffffffffu);

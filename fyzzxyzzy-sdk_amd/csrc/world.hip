@@ -1143,6 +1143,21 @@ __host__ __device__ inline void wake_record(fyzz_dy_body& b, bool queue = false)
     b.flags = (b.flags & ~3u) | (queue ? 8u : 0u);
 }
 
+// Scene::set_velocity / set_angular_velocity of a stepped world's body, on
+// the device: a record read back, edited and written takes two copies and
+// two synchronizations.
+struct VelocityEdit {
+    float linear[3], angular[3];
+    u32 set;  // bit0 linear, bit1 angular
+};
+__global__ void k_set_velocity(fyzz_dy_body* b, VelocityEdit e) {
+    for (int k = 0; k < 3; ++k) {
+        if (e.set & 1u) b->linear_velocity[k] = e.linear[k];
+        if (e.set & 2u) b->angular_velocity[k] = e.angular[k];
+    }
+    if (e.set) wake_record(*b);
+}
+
 // Scene::set_pose's invalidations (scene.cpp:651-700) for the box in
 // `slot`: every current broadphase pair holding it and its plane pair
 // lose their PCM cache (ShapeInteraction::resetManagerCachedState). When
@@ -1261,7 +1276,7 @@ struct fyzz_hip_world {
     DevBuf<u64> scene_pairs[2];
     // contact events
     bool notify = false;
-    DevBuf<u32> shape, touch_bb[2], touch_pl, slot_mgr, s1, s2, s3, ev_counts, ev_src, ev_pts, ev_off, d_npts;
+    DevBuf<u32> shape, touch_bb[2], touch_pl, slot_mgr, s1, s2, s3, ev_counts, ev_src, ev_pts, ev_off;
     DevBuf<u64> k1, k2, k3;
     DevBuf<fyzz_contact_event> events;
     DevBuf<fyzz_contact_event_point> points;
@@ -1587,11 +1602,10 @@ void reserve_events(fyzz_hip_world* w) {
         w->ev_tmp_vals.reserve(cap);
         w->ev_sort_scratch.reserve(sap::sort_keys_scratch_words(cap));
     }
-    w->ev_counts.reserve(4);
+    w->ev_counts.reserve(5);  // streams 1-3, events, points
     w->ev_src.reserve(w->ev_cap);
     w->ev_pts.reserve(w->ev_cap);
     w->ev_off.reserve(w->ev_cap);
-    w->d_npts.reserve(1);
     w->events.reserve(w->ev_cap);
     w->points.reserve(w->pt_cap);
 }
@@ -1611,8 +1625,8 @@ void publish_events(fyzz_hip_world* w, const sap::Lists& L, int c_prev, int c_cu
                        w->d_nm.p, w->mgr_cap, w->mgr_slot.p, w->slot_mgr.p);
     sel::select(st, cap, L.d_cur, EvPred1{A}, EvWrite1{A, w->k1.p, w->s1.p}, w->tiles.p, w->ev_counts.p);
     if (w->has_floor) {
-        hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, w->d_npts.p, 1u, n);
-        sel::select(st, n, w->d_npts.p, EvPred2{A}, EvWrite2{A, w->k2.p, w->s2.p}, w->tiles.p, w->ev_counts.p + 1);
+        hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, w->ev_counts.p + 4, 1u, n);
+        sel::select(st, n, w->ev_counts.p + 4, EvPred2{A}, EvWrite2{A, w->k2.p, w->s2.p}, w->tiles.p, w->ev_counts.p + 1);
     } else {
         hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, w->ev_counts.p + 1, 1u, 0u);
     }
@@ -1629,7 +1643,7 @@ void publish_events(fyzz_hip_world* w, const sap::Lists& L, int c_prev, int c_cu
     const u32 grid = std::min<u32>(grid_for(w->ev_cap, 256), 2048u);
     hipLaunchKernelGGL(k_ev_merge, dim3(grid), dim3(256), 0, st, A, w->events.p, w->ev_src.p, w->ev_pts.p);
     sel::exclusive_scan(st, w->ev_cap, w->ev_counts.p + 3, EvCount{w->ev_pts.p}, w->ev_off.p, w->tiles.p,
-                        w->d_npts.p);
+                        w->ev_counts.p + 4);
     hipLaunchKernelGGL(k_ev_points, dim3(grid), dim3(256), 0, st, A, w->ev_src.p, w->ev_off.p, w->events.p,
                        w->points.p, w->slot_mgr.p, w->managers.p, w->impulses.p, w->pt_cap);
     FYZZ_HIP_CHECK(hipGetLastError());
@@ -2040,9 +2054,7 @@ sap::Lists current_lists(fyzz_hip_world* w) {
 // the world's stream (authoring calls are host API calls, not step work).
 fyzz_dy_body read_body(fyzz_hip_world* w, u32 slot) {
     fyzz_dy_body b{};
-    hipStream_t st = w->ctx->stream;
-    FYZZ_HIP_CHECK(hipMemcpyAsync(&b, w->bodies.p + slot, sizeof b, hipMemcpyDeviceToHost, st));
-    FYZZ_HIP_CHECK(hipStreamSynchronize(st));
+    read_back(w->ctx, {{&b, w->bodies.p + slot, sizeof b}});
     return b;
 }
 
@@ -2052,11 +2064,14 @@ void write_body(fyzz_hip_world* w, u32 slot, const fyzz_dy_body& b) {
     FYZZ_HIP_CHECK(hipStreamSynchronize(st));
 }
 
+void require_editable(const fyzz_hip_world* w) {
+    FYZZ_REQUIRE(!(w->uploaded && w->native_order), kLogicError,
+                 "world: the native solver order takes no body edits after the first step");
+}
 // The record a setter edits: the host copy before the first step, the
 // device's afterwards (written back by commit_body).
 fyzz_dy_body& edit_body(fyzz_hip_world* w, u32 id, fyzz_dy_body& scratch_copy, u32* slot_out) {
-    FYZZ_REQUIRE(!(w->uploaded && w->native_order), kLogicError,
-                 "world: the native solver order takes no body edits after the first step");
+    require_editable(w);
     fyzz_dy_body& host = w->body(id);
     const u32 slot = static_cast<u32>(w->slot_of_id[id]);
     if (slot_out) *slot_out = slot;
@@ -2424,15 +2439,28 @@ int fyzz_hip_world_set_body_velocity(fyzz_hip_world* w, uint32_t body_id, const 
             FYZZ_REQUIRE(!angular || std::isfinite(angular[k]), kInvalidArgument,
                          "world: angular velocity must be finite");
         }
-        fyzz_dy_body tmp;
-        u32 slot = 0;
-        fyzz_dy_body& b = edit_body(w, body_id, tmp, &slot);
+        if (w->uploaded) {
+            require_editable(w);
+            (void)w->body(body_id);  // a dynamic body
+            world::VelocityEdit e{};
+            for (int k = 0; k < 3; ++k) {
+                if (linear) e.linear[k] = linear[k];
+                if (angular) e.angular[k] = angular[k];
+            }
+            e.set = (linear ? 1u : 0u) | (angular ? 2u : 0u);
+            hipLaunchKernelGGL(world::k_set_velocity, dim3(1), dim3(1), 0, w->ctx->stream,
+                               w->bodies.p + w->slot_of_id[body_id], e);
+            FYZZ_HIP_CHECK(hipGetLastError());
+            // in place when the call returns, whichever stream steps next
+            FYZZ_HIP_CHECK(hipStreamSynchronize(w->ctx->stream));
+            return;
+        }
+        fyzz_dy_body& b = w->body(body_id);
         for (int k = 0; k < 3; ++k) {
             if (linear) b.linear_velocity[k] = linear[k];
             if (angular) b.angular_velocity[k] = angular[k];
         }
         if (linear || angular) world::wake_record(b);
-        commit_body(w, slot, b);
     });
 }
 
@@ -2536,9 +2564,7 @@ int fyzz_hip_world_body_records(fyzz_hip_world* w, fyzz_dy_body* out, uint32_t c
             std::copy(w->host_bodies.begin(), w->host_bodies.begin() + m, out);
             return;
         }
-        FYZZ_HIP_CHECK(hipMemcpyAsync(out, w->bodies.p, sizeof(fyzz_dy_body) * m, hipMemcpyDeviceToHost,
-                                      w->ctx->stream));
-        FYZZ_HIP_CHECK(hipStreamSynchronize(w->ctx->stream));
+        read_back(w->ctx, {{out, w->bodies.p, sizeof(fyzz_dy_body) * m}});
     });
 }
 
@@ -2683,24 +2709,17 @@ int fyzz_hip_world_contact_events(fyzz_hip_world* w, fyzz_contact_event* events,
                                   uint32_t* n_points) {
     if (!w) return kInvalidArgument;
     return guarded(w->ctx, [&] {
-        u32 counts[4] = {0, 0, 0, 0}, np = 0;
-        hipStream_t st = w->ctx->stream;
-        if (w->notify && w->ev_cap && w->uploaded) {
-            FYZZ_HIP_CHECK(hipMemcpyAsync(counts, w->ev_counts.p, sizeof counts, hipMemcpyDeviceToHost, st));
-            FYZZ_HIP_CHECK(hipMemcpyAsync(&np, w->d_npts.p, 4, hipMemcpyDeviceToHost, st));
-            FYZZ_HIP_CHECK(hipStreamSynchronize(st));
-        }
+        u32 counts[5] = {0, 0, 0, 0, 0};
+        const bool live = w->notify && w->ev_cap && w->uploaded;
+        if (live) read_back(w->ctx, {{counts, w->ev_counts.p, sizeof counts}});
+        const u32 np = counts[4];
         FYZZ_REQUIRE(np <= w->pt_cap || !w->notify, kOverflow, "world: contact event points exceed capacity");
         if (n_events) *n_events = counts[3];
         if (n_points) *n_points = np;
-        const u32 ne = std::min(counts[3], capacity), mp = std::min(np, point_capacity);
-        if (events && ne)
-            FYZZ_HIP_CHECK(hipMemcpyAsync(events, w->events.p, sizeof(fyzz_contact_event) * ne, hipMemcpyDeviceToHost,
-                                          st));
-        if (points && mp)
-            FYZZ_HIP_CHECK(hipMemcpyAsync(points, w->points.p, sizeof(fyzz_contact_event_point) * mp,
-                                          hipMemcpyDeviceToHost, st));
-        FYZZ_HIP_CHECK(hipStreamSynchronize(st));
+        const u32 ne = events ? std::min(counts[3], capacity) : 0u, mp = points ? std::min(np, point_capacity) : 0u;
+        if (!live || ne || mp)
+            read_back(w->ctx, {{events, w->events.p, sizeof(fyzz_contact_event) * ne},
+                               {points, w->points.p, sizeof(fyzz_contact_event_point) * mp}});
     });
 }
 
