@@ -129,9 +129,7 @@ __device__ inline uint2 coarse_other(const uint4 c, u32 axis) {
 // 3 + axis; tiles of kSplitTile positions.
 constexpr u32 kSplitTile = 1024;  // 256 threads x 4 positions
 struct SplitArrays {
-    u32* key;      // [2 arrays][3 axes][2 kinds][n]
-    u32* pay;
-    uint2* cs;
+    uint4* entry;  // [2 arrays][3 axes][2 kinds][n]: key, payload, coarse bounds of the two other axes
     u32* pos;      // [2 arrays][3 axes][2n]
     u32* tile_max; // [6][tiles] max endpoints per tile
 };
@@ -190,9 +188,8 @@ __global__ __launch_bounds__(256) void k_split(u32 n2, const u32* new_key, const
             const u32 idx = kind ? mx : j - mx;
             S.pos[static_cast<std::size_t>(seg) * n2 + j] = idx;
             const std::size_t o = split_off(seg, kind, n) + idx;
-            S.key[o] = kk[k];
-            S.pay[o] = pe[k];
-            S.cs[o] = coarse_other(coarse[pe[k] >> 1], axis);
+            const uint2 cs = coarse_other(coarse[pe[k] >> 1], axis);
+            S.entry[o] = make_uint4(kk[k], pe[k], cs.x, cs.y);
             mx += kind;
         }
         __syncthreads();
@@ -462,65 +459,82 @@ __global__ __launch_bounds__(256) void k_cross(CrossArgs A) {
 // The same walks when the arrays were split by kind this frame (a settling
 // pile: most boxes move and the walks are long). A walk scans the other
 // kind's array from the walker's place in the sorted order; each step reads
-// the entry's key, payload and the gathered bounds of the two other axes in
-// sequence; only candidates that pass them touch per-slot data.
+// one entry: key, payload and the gathered bounds of the two other axes;
+// only candidates that pass them touch per-slot data.
 struct SplitWalk {
-    const u32* K;
-    const u32* P;
-    const uint2* C;
+    const uint4* E;
     u32 start;  // walking up: the first other-kind index after the walker; down: one past the last before it
-    u32 n;
+    u32 left;   // entries from there to the array's end
 };
-__device__ inline bool walk_inside_s(const WalkGeom& g, const SplitWalk& sw, u32 step, u32& pj, uint2& cj) {
-    if (g.up) {
-        const u32 j = sw.start + step - 1u;
-        if (j >= sw.n) return false;
-        const u32 kj = sw.K[j];
-        pj = sw.P[j];
-        cj = sw.C[j];
-        return kj < g.bound_v || (kj == g.bound_v && pj < g.pe);
-    }
-    if (step > sw.start) return false;
-    const u32 j = sw.start - step;
-    const u32 kj = sw.K[j];
-    pj = sw.P[j];
-    cj = sw.C[j];
-    return kj > g.bound_v || (kj == g.bound_v && pj > g.pe);
+// the step-th entry of the walk, step in 1..left
+__device__ inline uint4 walk_entry(const WalkGeom& g, const SplitWalk& sw, u32 step) {
+    return sw.E[g.up ? sw.start + step - 1u : sw.start - step];
 }
-__device__ inline SplitWalk split_walk(const CrossArgs& A, const Walk& w, u32 own) {
+__device__ inline bool walk_inside_s(const WalkGeom& g, const uint4& e) {
+    return g.up ? e.x < g.bound_v || (e.x == g.bound_v && e.y < g.pe)
+                : e.x > g.bound_v || (e.x == g.bound_v && e.y > g.pe);
+}
+__device__ inline SplitWalk split_walk(const CrossArgs& A, const Walk& w, const WalkGeom& g, u32 own) {
     const u32 seg = w.arr * 3u + w.axis, n = A.n2 >> 1;
-    const u32 other = w.kind ^ 1u;
-    const std::size_t o = split_off(seg, other, n);
     SplitWalk sw;
-    sw.K = A.split.key + o;
-    sw.P = A.split.pay + o;
-    sw.C = A.split.cs + o;
-    sw.n = n;
+    sw.E = A.split.entry + split_off(seg, w.kind ^ 1u, n);
     // other-kind entries before the walker = own - (same-kind entries before it)
     sw.start = own - A.split.pos[static_cast<std::size_t>(seg) * A.n2 + own];
+    sw.left = g.up ? n - sw.start : sw.start;
     return sw;
 }
-// ca: the walker's own coarse bounds on the same two axes (its old and new
-// keys); a candidate that misses them on one of them cannot change status.
-__device__ inline void walk_visit_g(const CrossArgs& A, const Walk& w, u32 pf, const uint2& cb, const uint2& ca,
-                                    const Rec& an, const Rec& ao) {
-    const u32 b = pf >> 1;
-    if ((pf & 1u) == w.kind || b == w.a || !coarse_overlap2(ca, cb)) return;
+// The walks' candidates, queued per wave: the re-test of one is a chain of
+// scattered reads, and with a candidate on some lane at nearly every step
+// the whole wave would wait for it each time. Queued, 64 of them are tested
+// at once: with one 16-byte entry per step, four read ahead, and this queue a
+// formed pile of 100,000 boxes takes 230 us instead of 346 (280 without the
+// queue), a heap of 20,011 47 instead of 105. What bounds it is the
+// longest of a wave's 64 walks (up to kShortWalkG entries).
+struct WalkQueue {
+    u64* q;   // LDS, 2 * kWave entries: walker << 33 | array << 32 | candidate
+    u32 n;    // queued (the same on every lane)
+};
+__device__ inline void walk_test(const CrossArgs& A, u64 x) {
+    const u32 a = static_cast<u32>(x >> 33), b = static_cast<u32>(x);
     const bool b_moved = (A.moved_bits[b >> 5] >> (b & 31u)) & 1u;
     // an unmoved endpoint sits at the same value in both arrays: the
     // new-array walk already saw it
-    if (b_moved || !w.arr) {
-        const Rec bn = A.cur[b];
-        if (pair_allowed(an, bn)) {
-            const Rec bo = b_moved ? A.prev[b] : bn;
-            const bool ov_new = overlap3(an, bn);
-            const bool ov_old = overlap3(ao, bo);
-            if (ov_new != ov_old) emit(pair_key(w.a, b) | (ov_new ? kFoundBit : 0ull), A.out, A.cnt, kDelta, A.cap);
-        }
+    if (!b_moved && ((x >> 32) & 1u)) return;
+    const Rec an = A.cur[a], bn = A.cur[b];
+    if (!pair_allowed(an, bn)) return;
+    const bool ov_new = overlap3(an, bn);
+    const bool ov_old = overlap3(A.prev[a], b_moved ? A.prev[b] : bn);
+    if (ov_new != ov_old) emit(pair_key(a, b) | (ov_new ? kFoundBit : 0ull), A.out, A.cnt, kDelta, A.cap);
+}
+// (all lanes of the wave take part in both)
+__device__ inline void walk_flush(const CrossArgs& A, WalkQueue& Q, u32 least) {
+    while (Q.n >= least && Q.n) {
+        const u32 m = min(Q.n, static_cast<u32>(kWave));
+        Q.n -= m;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (lane_id() < m) walk_test(A, Q.q[Q.n + lane_id()]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
 }
-// Entries a gathered walk's thread takes before handing the rest to a wave.
+// ca: the walker's own coarse bounds on the same two axes (its old and new
+// keys); a candidate that misses them on one of them cannot change status.
+__device__ inline void walk_visit_g(const CrossArgs& A, WalkQueue& Q, bool live, const Walk& w, const uint4& e,
+                                    const uint2& ca) {
+    const u32 b = e.y >> 1;
+    const bool hit = live && b != w.a && coarse_overlap2(ca, make_uint2(e.z, e.w));
+    const u64 mask = __ballot(hit);
+    if (!mask) return;
+    if (hit)
+        Q.q[Q.n + static_cast<u32>(__popcll(mask & ((1ull << lane_id()) - 1ull)))] =
+            static_cast<u64>(w.a) << 33 | static_cast<u64>(w.arr) << 32 | b;
+    Q.n += static_cast<u32>(__popcll(mask));
+    walk_flush(A, Q, kWave);
+}
+// Entries a gathered walk's thread takes before handing the rest to a wave
+// (fewer make more long walks, whose list takes one counter: 128 entries 288
+// us with the pile's long walks, 256 252, 32 428).
 constexpr u32 kShortWalkG = 256;
+constexpr u32 kWalkAhead = 4;  // entries read at once (2: 248 us on the pile, 8: 229)
 // Gathered walks are issued in sorted order: work item t is position j of
 // array (arr, axis), t = (arr * 3 + axis) * n2 + j, and walks when its
 // endpoint belongs to a moved box. Neighbouring lanes then walk
@@ -540,36 +554,55 @@ __device__ inline WalkGeom walk_geom_at(const Walk& w, u32 v_old, u32 v_new) {
     return {w.arr ? v_new : v_old, (w.a << 1) | w.kind, (w.arr != 0) == (v_new > v_old)};  // old array: toward v_new
 }
 __global__ __launch_bounds__(256) void k_cross_g(CrossArgs A) {
+    __shared__ u64 queue[256 / kWave][2 * kWave];
+    WalkQueue Q{queue[threadIdx.x / kWave], 0u};
     const u32 n_work = 6u * A.n2;
-    for (u32 t = blockIdx.x * blockDim.x + threadIdx.x; t < n_work; t += gridDim.x * blockDim.x) {
-        Walk w;
-        u32 own;
-        if (!walker_at(A, t, w, own)) continue;
-        const Rec an = A.cur[w.a];
-        const Rec ao = A.prev[w.a];
-        const u32 v_old = ao.k[w.axis + 3 * w.kind];
-        const u32 v_new = an.k[w.axis + 3 * w.kind];
-        if (v_old == v_new) continue;
-        const WalkGeom g = walk_geom_at(w, v_old, v_new);
-        const SplitWalk sw = split_walk(A, w, own);
-        const uint2 ca = coarse_other(A.coarse[w.a], w.axis);
-        for (u32 step = 1;; ++step) {
-            u32 pj = 0;
-            uint2 cj;
-            if (!walk_inside_s(g, sw, step, pj, cj)) break;
-            walk_visit_g(A, w, pj, cj, ca, an, ao);
-            if (step == kShortWalkG) {
-                const u32 slot = atomicAdd(&A.cnt[kLongWalks], 1u);
-                if (slot < A.long_cap)
-                    A.long_walks[slot] = t;
-                else
-                    atomicOr(&A.cnt[kOverflow], 4u);
+    const u32 lane = lane_id();
+    for (u32 base = blockIdx.x * blockDim.x + threadIdx.x - lane; base < n_work; base += gridDim.x * blockDim.x) {
+        const u32 t = base + lane;
+        Walk w{};
+        u32 own = 0;
+        WalkGeom g{};
+        SplitWalk sw{};
+        uint2 ca = make_uint2(0u, 0u);
+        bool more = t < n_work && walker_at(A, t, w, own);
+        if (more) {
+            const u32 v_old = A.prev[w.a].k[w.axis + 3 * w.kind], v_new = A.cur[w.a].k[w.axis + 3 * w.kind];
+            more = v_old != v_new;
+            if (more) {
+                g = walk_geom_at(w, v_old, v_new);
+                sw = split_walk(A, w, g, own);
+                ca = coarse_other(A.coarse[w.a], w.axis);
+                more = sw.left != 0u;
+            }
+        }
+        for (u32 done = 0; __ballot(more); done += kWalkAhead) {
+            if (done == kShortWalkG) {
+                if (more) {
+                    const u32 slot = atomicAdd(&A.cnt[kLongWalks], 1u);
+                    if (slot < A.long_cap)
+                        A.long_walks[slot] = t;
+                    else
+                        atomicOr(&A.cnt[kOverflow], 4u);
+                }
                 break;
+            }
+            uint4 e[kWalkAhead];
+#pragma unroll
+            for (u32 k = 0; k < kWalkAhead; ++k)
+                if (more) e[k] = walk_entry(g, sw, min(done + 1u + k, sw.left));
+#pragma unroll
+            for (u32 k = 0; k < kWalkAhead; ++k) {
+                more = more && done + k < sw.left && walk_inside_s(g, e[k]);
+                walk_visit_g(A, Q, more, w, e[k], ca);
             }
         }
     }
+    walk_flush(A, Q, 1u);
 }
 __global__ __launch_bounds__(256) void k_cross_long_g(CrossArgs A) {
+    __shared__ u64 queue[256 / kWave][2 * kWave];
+    WalkQueue Q{queue[threadIdx.x / kWave], 0u};
     const u32 lane = lane_id();
     const u32 n_long = min(A.cnt[kLongWalks], A.long_cap);
     const u32 n_waves = gridDim.x * (blockDim.x / kWave);
@@ -578,19 +611,19 @@ __global__ __launch_bounds__(256) void k_cross_long_g(CrossArgs A) {
         Walk w;
         u32 own;
         (void)walker_at(A, t, w, own);
-        const Rec an = A.cur[w.a];
-        const Rec ao = A.prev[w.a];
-        const WalkGeom g = walk_geom_at(w, ao.k[w.axis + 3 * w.kind], an.k[w.axis + 3 * w.kind]);
-        const SplitWalk sw = split_walk(A, w, own);
+        const u32 v_old = A.prev[w.a].k[w.axis + 3 * w.kind], v_new = A.cur[w.a].k[w.axis + 3 * w.kind];
+        const WalkGeom g = walk_geom_at(w, v_old, v_new);
+        const SplitWalk sw = split_walk(A, w, g, own);
         const uint2 ca = coarse_other(A.coarse[w.a], w.axis);
         for (u32 base = kShortWalkG;; base += kWave) {
-            u32 pj = 0;
-            uint2 cj = make_uint2(0, 0);
-            const bool inside = walk_inside_s(g, sw, base + lane + 1, pj, cj);
-            if (inside) walk_visit_g(A, w, pj, cj, ca, an, ao);
+            const u32 step = base + lane + 1u;
+            const uint4 e = walk_entry(g, sw, min(step, sw.left));
+            const bool inside = step <= sw.left && walk_inside_s(g, e);
+            walk_visit_g(A, Q, inside, w, e, ca);
             if (__ballot(inside) != ~0ull) break;
         }
     }
+    walk_flush(A, Q, 1u);
 }
 
 // ---- compaction predicates / writers ----
@@ -981,8 +1014,8 @@ struct Sap {
         radix_counts, radix_totals, sel_tiles, dummy_a, dummy_b;
     DevBuf<Rec> rec_cur, rec_prev;
     DevBuf<uint4> coarse;
-    DevBuf<u32> split_key, split_pay, split_pos, split_tiles;  // the gathered walks' kind-split arrays
-    DevBuf<uint2> split_cs;
+    DevBuf<uint4> split_entry;  // the gathered walks' kind-split arrays
+    DevBuf<u32> split_pos, split_tiles;
     DevBuf<u32> list_bar;          // grid barrier and totals of k_lists
     DevBuf<u64> pairs[2], work_a, work_b, found, lost, kept;
     DevBuf<u32> src;         // previous-list index of each current pair (incremental frames)
@@ -1101,7 +1134,7 @@ void advance(Sap& s, const float* pos, const float* quat, const float* half, con
         // of them are listed (a settling pile). Otherwise the walks load
         // each candidate's bounds by slot.
         const bool gather = n && (!dirty || 2ull * n_dirty >= n);
-        const SplitArrays split{s.split_key.p, s.split_pay.p, s.split_cs.p, s.split_pos.p, s.split_tiles.p};
+        const SplitArrays split{s.split_entry.p, s.split_pos.p, s.split_tiles.p};
         // per-slot walks start from their endpoint's position in each array
         // (the SapBox1D min/max indices of the reference GPU path), for the
         // moved boxes only; the sorted-order walks start at their position
@@ -1277,9 +1310,7 @@ int fyzz_hip_sap_create(fyzz_hip_context* ctx, uint32_t n, const uint32_t* body_
         s.rec_prev.reserve(n);
         s.coarse.reserve(n);
         // kind-split arrays of both sorted arrays: 2 x 3 x 2n entries each
-        s.split_key.reserve(6ull * n2);
-        s.split_pay.reserve(6ull * n2);
-        s.split_cs.reserve(6ull * n2);
+        s.split_entry.reserve(6ull * n2);
         s.split_pos.reserve(6ull * n2);
         s.split_tiles.reserve(6ull * ((n2 + sap::kSplitTile - 1) / sap::kSplitTile) + 1);
         s.list_bar.reserve(sap::kListBarWords);

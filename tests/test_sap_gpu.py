@@ -200,6 +200,13 @@ def test_incremental_sap_all_moving(ctx, orc, torch_cuda):
     _run_frames(ctx, orc, torch_cuda, 8000, 4, 10, 1.5, 8.0, 1.0, False)
 
 
+@pytest.mark.parametrize("n,move", [(33, 4.0), (64, 0.2), (65, 40.0), (700, 40.0), (3001, 20.0)])
+def test_gathered_walks_queue_edges(ctx, orc, torch_cuda, n, move):
+    # all boxes move: queues that never fill, that fill in one step, and (far
+    # moves) walks past the entries one thread takes
+    _run_frames(ctx, orc, torch_cuda, n, 3, 21, 1.2, move, 1.0, False, delta_capacity=1_000_000)
+
+
 @pytest.mark.parametrize("force_full", [(), (2,), (3,)])
 @pytest.mark.parametrize("tight", [False, True])
 def test_counts_of_published_and_copied_frames_agree(ctx, torch_cuda, force_full, tight):
