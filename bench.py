@@ -66,12 +66,9 @@ DT = 1.0 / 120.0
 
 # HBM bytes per launch from rocprofv3 PMC passes (FETCH_SIZE x 2.0 and
 # WRITE_SIZE x 1.0 after the plain-copy calibration), keyed by stage; the
-# passes and the launches they cover are in profiles/pile_100k_counters.md
-# and profiles/sap_1m_incremental.md.
-PILE_TRAFFIC = {
-    "dy.pgs": {"bytes": 2_235_000_000, "algorithmic_bytes": 543_700_000,
-               "measured_on": "formed pile: 3 steps after loading the state saved at step 645 (248k managers)"},
-}
+# passes and the launches they cover are in profiles/sap_1m_incremental.md.
+# (The pile's sweep has no entry: its row layout is newer than the passes.)
+PILE_TRAFFIC = {}
 SAP_SORT_TRAFFIC_BYTES = 611_000_000
 
 
@@ -106,7 +103,7 @@ def parse():
     p.add_argument("--eager", action="store_true",
                    help="pile: direct launches only (no graph capture; for counter passes)")
     p.add_argument("--plain-launch", action="store_true",
-                   help="plain instead of cooperative launches of the Dy grid-barrier kernels (counter profilers)")
+                   help="plain instead of cooperative launches of the Dy sweep kernels (counter profilers)")
     p.add_argument("--calibrate-copy", action="store_true",
                    help="run one plain 256 MiB device copy first (PMC byte-counter calibration)")
     return p.parse_args()

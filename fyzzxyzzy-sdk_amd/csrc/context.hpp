@@ -124,7 +124,7 @@ struct Readback {
 struct fyzz_hip_context {
     int device = 0;
     hipStream_t stream = nullptr;  // null = the device's default stream
-    bool cooperative = true;       // grid-barrier kernels: cooperative or plain launches
+    bool cooperative = true;       // the Dy sweeps: cooperative or plain launches
     std::string last_error;
     fyzz_hip::Profiler prof;
     fyzz_hip::HostStage stage;

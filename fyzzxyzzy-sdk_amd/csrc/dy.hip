@@ -12,7 +12,7 @@
 //   cached_friction_patch_valid                 3981-4010     history_valid
 //   solve_constraint_task                       8853-9148     k_pgs
 //   publish_solver_bodies, integrate_solver_task, integrate_quaternion
-//                                               9509-9549, 10508-10707, 111-146   k_integrate
+//                                               9509-9549, 10508-10707, 111-146   integrate_body, in k_outputs
 //
 // Admitted scene class: dynamic boxes and static planes/boxes, PCM
 // manifolds (one normal per manager, 1-4 contacts), non-compliant
@@ -23,9 +23,8 @@
 // sequential first-fit over 32-bit masks exactly: a manager's partition
 // depends only on the masks its two bodies carry after the earlier managers
 // incident to them, so a manager is coloured as soon as its predecessor on
-// each body is (one cooperative launch, no global rounds). Within a
-// partition no two managers share a
-// dynamic body and the static world's solver body keeps a zero state, so
+// each body is (one launch, no global rounds). Within a partition no two
+// managers share a dynamic body and the static world's solver body keeps a zero state, so
 // solving a partition's managers concurrently gives the sequential sweep's
 // values bit for bit.
 #include <hip/hip_runtime.h>
@@ -335,19 +334,16 @@ __global__ __launch_bounds__(kBlock) void k_rows(Ws W) {
 
 // ------------------------------------------------------------ partitions
 
-__device__ inline bool dyn_dyn(const fyzz_dy_manager& M) { return M.body0 >= 0 && M.body1 >= 0; }
-
 // First-fit partitions over 32-bit masks (scene.cpp:7352-7445) for one task
 // spanning the manager list; stable scatter by partition (7447-7489).
 //
 // The data-parallel phases are plain kernels over bodies or managers:
-// degrees, their scan, incidence lists (CSR by body), each body's list in
-// manager order with the predecessor of every dynamic/dynamic entry,
-// static managers after the body's dynamic partitions, sizes, offsets and
-// the scatter. The colouring is one cooperative kernel: a manager's
-// partition depends only on the masks its two bodies carry after their
-// earlier managers, so each thread walks its managers in increasing order
-// (m = tid, tid + threads, ...) and colours one as soon as the entries of
+// degrees, incidence lists by body, each body's list in manager order with
+// the predecessor of every dynamic/dynamic entry, static managers after the
+// body's dynamic partitions, sizes, offsets and the scatter. The colouring
+// is one kernel: a manager's partition depends only on the masks its two
+// bodies carry after their earlier managers, so workgroups draw tiles of
+// managers in increasing order and colour one as soon as the entries of
 // its two predecessors are published. An entry is one 64-bit word (ready
 // bit, chain level, mask after the manager) written and read as a single
 // relaxed agent-scope atomic, cleared by the degree kernel every step. The
@@ -2219,8 +2215,8 @@ int resident_blocks(const void* kernel, int device) {
 }
 // Cooperative launch (the runtime checks that every workgroup is resident).
 // Inside a captured graph the kernels are launched as plain kernels with
-// the same small grid (far below the device's resident capacity); the grid
-// barrier's bounded spin turns a non-resident grid into a status flag.
+// the same small grid (far below the device's resident capacity); the
+// sweep's bounded waits turn a non-resident grid into a status flag.
 void launch_coop(const void* kernel, int blocks, dy::Ws& ws, hipStream_t st, bool plain) {
     void* args[] = {&ws};
     if (plain)

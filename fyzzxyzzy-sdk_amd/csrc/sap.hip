@@ -17,9 +17,9 @@
 //   sorted[2][3][2n]   (key, payload) per axis, current and previous frame;
 //                      payload = slot << 1 | is_max
 //   split[2][3][2][n]  gathered walks only: each sorted array split by
-//                      endpoint kind (key, payload, coarse bounds of the
-//                      other two axes), with each position's index in its
-//                      kind's array
+//                      endpoint kind (one 16-B entry: key, payload, coarse
+//                      bounds of the other two axes), with each position's
+//                      index in its kind's array
 //   pairs[2][cap]      sorted u64 (lo slot << 32 | hi slot)
 // Boxes are identified by slot (0..n-1, increasing shape id), so slot
 // order is shape-id order and every tie-break matches the reference.

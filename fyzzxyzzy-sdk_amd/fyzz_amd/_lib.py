@@ -177,7 +177,7 @@ class Context:
         self.call("fyzz_hip_synchronize")
 
     def set_cooperative(self, cooperative: bool = True):
-        """Cooperative (default) or plain launches of the Dy grid-barrier
+        """Cooperative (default) or plain launches of the Dy sweep
         kernels; results are identical."""
         self.call("fyzz_hip_set_cooperative", 1 if cooperative else 0)
 

@@ -141,7 +141,7 @@ const char* fyzz_hip_last_error(const fyzz_hip_context* ctx);
  * default stream. */
 int fyzz_hip_set_stream(fyzz_hip_context* ctx, void* hip_stream);
 int fyzz_hip_synchronize(fyzz_hip_context* ctx);
-/* Launch mode of the Dy grid-barrier kernels (no counterpart in the
+/* Launch mode of the Dy sweeps (k_pgs, k_pgs_adjoint; no counterpart in the
  * reference): cooperative != 0 (default) uses hipLaunchCooperativeKernel,
  * which checks that every workgroup is resident; 0 launches the same
  * resident-sized grid as a plain kernel, as inside captured graphs (for
